@@ -14,10 +14,6 @@
 //   V cache       [layer][kv_head][max_seq][128]        (as qwen3.h:62-76)
 //   rope tables   [max_seq][64] cos and sin, built on the host with the
 //                 reference formula (ops_scalar.c:21-35)
-// The chunk attention keeps its tokens' scores in LDS, sized by the chunk's
-// context: up to 69 KB at QM_MAX_SEQ with one token per block, above the
-// default 64 KB limit, which it raises once.
-#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -28,6 +24,7 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
 #define WAVE 64
 #define NTH 256
@@ -172,200 +169,327 @@ __global__ __launch_bounds__(NTH) void k_rows_norm(float *__restrict__ x, const 
 
 // ---------------------------------------------------------------------------
 // Chunk of nt tokens at positions pos0 .. pos0+nt-1 (pos0 = *pos_d), step 1:
-// QK-norm (qwen3.c:298-305) then RoPE (ops_scalar.c:21-35) of every q and k
-// head; q is written back in place, k and v go to the KV cache entry of
-// their position (qwen3.c:497-512).  grid = (nt, 6): block (i, b), wave w
-// handles row 4b + w of token i (rows 0-15 q heads, 16-23 k heads + v copy).
+// QK-norm (qwen3.c:298-305) then RoPE (ops_scalar.c:21-35) of every k head;
+// k and v go to the KV cache entry of their position (qwen3.c:497-512).
+// grid = (nt, 2): block (i, b), wave w handles kv head 4b + w of token i.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(NTH) void k_qk_rope_cache(float *__restrict__ qkv, float *__restrict__ kc,
-                                                       float *__restrict__ vc,
-                                                       const uint16_t *__restrict__ qn,
-                                                       const uint16_t *__restrict__ kn,
-                                                       const float *__restrict__ rcos,
-                                                       const float *__restrict__ rsin,
-                                                       const int *__restrict__ pos_d, int max_seq,
-                                                       float eps) {
+__global__ __launch_bounds__(NTH) void k_rope_cache(const float *__restrict__ qkv, float *__restrict__ kc,
+                                                    float *__restrict__ vc,
+                                                    const uint16_t *__restrict__ kn,
+                                                    const float *__restrict__ rcos,
+                                                    const float *__restrict__ rsin,
+                                                    const int *__restrict__ pos_d, int max_seq, float eps) {
     const int i = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int rr = blockIdx.y * 4 + wave;      // 0 .. 23
+    const int hd = blockIdx.y * 4 + wave;      // 0 .. 7
     const int pos = *pos_d + i;
     if (*pos_d < 0 || pos >= max_seq) return;
-    float *row = qkv + (size_t)i * QKV_LD;
-    const bool isq = rr < NKV * GRP;
-    const int hd = isq ? rr : rr - NKV * GRP;
-    float *src = isq ? row + (size_t)hd * HD : row + KOFF + (size_t)hd * HD;
-    const uint16_t *w = isq ? qn : kn;
+    const float *src = qkv + (size_t)i * QKV_LD + KOFF + (size_t)hd * HD;
+    const float *vs = qkv + (size_t)i * QKV_LD + VOFF + (size_t)hd * HD;
     const float x0 = src[lane], x1 = src[lane + 64];
-    const float w0 = bf16f(w[lane]), w1 = bf16f(w[lane + 64]);
+    const float v0 = vs[lane], v1 = vs[lane + 64];
+    const float w0 = bf16f(kn[lane]), w1 = bf16f(kn[lane + 64]);
     const float c = rcos[(size_t)pos * (HD / 2) + lane], sn = rsin[(size_t)pos * (HD / 2) + lane];
     const float ss = wave_sum(sumsq2(x0, x1));
     const float sc = 1.0f / sqrtf(ss / (float)HD + eps);
     const float y0 = (x0 * sc) * w0, y1 = (x1 * sc) * w1;
     float o0, o1;
     rope_pair(y0, y1, c, sn, o0, o1);
-    if (isq) {
-        src[lane] = o0;
-        src[lane + 64] = o1;
-    } else {
-        float *kb = kc + (size_t)hd * (HD / 4) * max_seq * 4;
-        kb[((size_t)(lane >> 2) * max_seq + pos) * 4 + (lane & 3)] = o0;
-        kb[((size_t)((lane + 64) >> 2) * max_seq + pos) * 4 + (lane & 3)] = o1;
-        float *vb = vc + ((size_t)hd * max_seq + pos) * HD;
-        const float *vs = row + VOFF + (size_t)hd * HD;
-        vb[lane] = vs[lane];
-        vb[lane + 64] = vs[lane + 64];
-    }
+    float *kb = kc + (size_t)hd * (HD / 4) * max_seq * 4;
+    kb[((size_t)(lane >> 2) * max_seq + pos) * 4 + (lane & 3)] = o0;
+    kb[((size_t)((lane + 64) >> 2) * max_seq + pos) * 4 + (lane & 3)] = o1;
+    float *vb = vc + ((size_t)hd * max_seq + pos) * HD;
+    vb[lane] = v0;
+    vb[lane + 64] = v1;
 }
 
 // ---------------------------------------------------------------------------
-// Chunk step 2: causal GQA attention (qwen3.c:377-436) for QT consecutive
-// tokens of the chunk and kv head g: block (b, g) takes tokens QT b ..
-// QT b + QT - 1 (those below nt) with their GRP query heads, R = QT GRP rows
-// (row r = token r / GRP, head r % GRP), roped q in qkv and every key/value
-// t <= pos0 + i in the cache (written by step 1).
-//   scores s[r][t] = q_r . k_t / sqrt(128); softmax over t (ops_scalar.c:
-//   37-44), normalised as there; out_r = sum_t p[r][t] v_t.
-// Every K and V row a block loads serves all R rows, so the cache traffic
-// of a chunk falls by QT.  Positions past a row's own context score -inf
-// and weigh 0: its max, sums and weighted V are those of a one-token block
-// bit for bit (only exact zeros are added, after its own positions).
-// grid = ceil(nt / QT) * NKV blocks, block b taking kv head b % NKV and tokens
-// QT (b / NKV) ..: blocks run on XCD b mod 8, so each XCD serves one head's K
-// and V from its own L2 (measured on MI355X against a (tokens, head) grid:
-// 128-token prefill 1.65 -> 1.62 ms, 2,014 tokens 39.7 -> 39.1 ms); 256 threads,
-// dynamic LDS =
-// qm_attention_lds_bytes(QT, ldp); ldp >= pos0 + nt is the score row stride.
+// Chunk step 2: causal GQA attention (qwen3.c:377-436) on the matrix cores in
+// fp32 (v_mfma_f32_16x16x4_f32: products and sums in fp32, as the scalar
+// code's), softmax over running maxima (ops_scalar.c:37-44 regrouped).
 // ---------------------------------------------------------------------------
-template <int QT>
-__global__ __launch_bounds__(NTH) void k_attention(const float *__restrict__ qkv,
-                                                   float *__restrict__ out,
-                                                   const float *__restrict__ kc,
-                                                   const float *__restrict__ vc,
-                                                   const int *__restrict__ pos_d, int nt, int max_seq,
-                                                   int ldp, float scale) {
-    constexpr int R = QT * GRP;
-    const int g = blockIdx.x % NKV, i0 = (int)(blockIdx.x / NKV) * QT, tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+// A block owns 8 MT consecutive tokens of kv head g with their GRP query
+// heads: MT tiles of 16 rows, row j of a tile = token j / 2, head j % 2.  Its
+// NW waves take the 16-position tiles of the context in turn (wave w of key
+// split y: tiles w + NW y, + NW KS, ...) and merge their partial softmaxes
+// through LDS; with KS key splits each block writes a partial that
+// k_attn_chunk_merge merges.  Every operand goes from memory straight into
+// the registers of its MFMA, only q through LDS:
+//   S^T = K Q^T   lane (c, h) = (lane % 16, lane / 16) loads the 16-byte
+//                 d-chunks 4s + h of key c: MFMA j of step s contracts dims
+//                 16s + 4h + j, for which it holds q row c in the same order
+//   O^T += V^T P^T  the accumulator of S^T holds keys 4h + r of q row c, which
+//                 is the B operand of the MFMA over keys 4h + r; V row 4h + r
+//                 is loaded as floats 8c .. 8c + 7, so output tile dt has dims
+//                 8i + dt and lane (c, h) ends with dims 32h .. 32h + 31 of
+//                 q row c, in order
+// The waves normalise and rope the block's query rows into LDS at entry (q of
+// step s: one 16-byte read per row tile).  The V loads of a tile are in flight
+// during its S product, the next tile's K loads during its P V product.
+// Positions past a row's own context score -inf and weigh 0; a V entry that
+// is not finite must not reach the rows that do not see it (0 * inf), so
+// tiles on the diagonal look for one and then keep such rows' sums apart.
+// grid = (ceil(nt / (8 MT)) * NKV, KS): block b takes kv head b % NKV, so each
+// XCD (b mod 8) serves one head's K and V from its own L2, and the token
+// tiles with the longest contexts first.
+// Bound by the fp32 matrix cores at long contexts (64 MFMAs of 32 cycles per
+// wave and tile) and by its chain of dependent loads at short ones.  Measured
+// on MI355X per launch against a VALU kernel with two tokens per block and
+// the scores in LDS: 128 tokens 11.6 -> 8.7 us, the 128-token chunks of an
+// 1,800-token prompt 40.0 -> 17.5 us (+ 4.3 for the merge), one token behind
+// 700 positions 28.2 -> 13.6 (+ 4.0).
+#define ATT_LD QM_ATT_PART             // row stride of a partial: 16-byte rows, conflict-free
+#define ATT_KS QM_ATT_KS               // key splits, at most
+
+// 1 / sqrt(head_dim), the constant of qwen3.c:311
+#define ATT_SCALE 0.08838834764831845f
+
+__device__ __forceinline__ bool not_finite(float x) { return (__float_as_uint(x) & 0x7F800000u) == 0x7F800000u; }
+
+template <int MT, int NW>
+__global__ __launch_bounds__(WAVE * NW, 2) void k_attn_chunk(const float *__restrict__ qkv,
+                                                             float *__restrict__ out, float *__restrict__ part,
+                                                             const float *__restrict__ kc,
+                                                             const float *__restrict__ vc,
+                                                             const uint16_t *__restrict__ qn,
+                                                             const float *__restrict__ rcos,
+                                                             const float *__restrict__ rsin,
+                                                             const int *__restrict__ pos_d, int nt, int max_seq,
+                                                             float eps) {
+    constexpr int TOK = 8 * MT, R = 16 * MT;             // tokens and rows of a block
+    const int g = blockIdx.x % NKV;
+    const int ntile = gridDim.x / NKV;
+    const int i0 = (ntile - 1 - (int)(blockIdx.x / NKV)) * TOK;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, h = lane >> 4;
     const int pos0 = *pos_d;
-    const int nq = min(QT, nt - i0);           // tokens of this block
-    const int ctxmax = pos0 + i0 + nq;         // context of its last token
-    // uniform per block, before any barrier
-    if (pos0 < 0 || nq <= 0 || ctxmax > max_seq || ctxmax > ldp) return;
+    const int nq = min(TOK, nt - i0);
+    const int ctx = pos0 + i0 + nq;                      // context of the block's last token
+    if (pos0 < 0 || nq <= 0 || ctx > max_seq) return;    // uniform per block, before any barrier
 
-    extern __shared__ float sm[];
-    float *sq = sm;                            // [R][HD]
-    float *red = sq + R * HD;                  // [4][R][HD] partial outputs
-    float *sred = red + 4 * R * HD;            // [R][4] block reductions
-    float *p = sred + 4 * R;                   // [R][ldp]
+    __shared__ __align__(16) float so[NW][R][ATT_LD];    // the waves' sums of e^(s - m) v
+    float (*sq)[ATT_LD] = so[0];                         // before them, the query rows
+    __shared__ float sm[NW][R], sl[NW][R];               // their maxima and sums of e^(s - m)
 
-    for (int e = tid; e < R * HD; e += NTH) {
-        const int r = e / HD, ti = i0 + r / GRP;
-        sq[e] = ti < nt ? qkv[(size_t)ti * QKV_LD + (size_t)(g * GRP + r % GRP) * HD + e % HD] : 0.0f;
+    const __amdgpu_buffer_rsrc_t rk = buf_rsrc(kc + (size_t)g * HD * max_seq, (size_t)HD * max_seq * 4);
+    const __amdgpu_buffer_rsrc_t rv = buf_rsrc(vc + (size_t)g * max_seq * HD, (size_t)max_seq * HD * 4);
+    const int nkt = (ctx + 15) >> 4, kstep = NW * gridDim.y;
+    int kt = wave + NW * blockIdx.y;
+    f32x4 kk[8], vv[4][2];
+    auto load_k = [&](int tile) {                        // tiles past the context read zeros
+        const int t = 16 * tile + c;
+        const uint32_t off = t < ctx ? (uint32_t)((h * max_seq + t) * 16) : BUF_OOB;
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            kk[s] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + (uint32_t)(s * 64) * max_seq, 0, 0));
+    };
+    load_k(kt);
+
+    // the block's query rows, shared by its waves: QK-norm and RoPE (rows past
+    // nt are zeros)
+    {
+        const float w0 = bf16f(qn[lane]), w1 = bf16f(qn[lane + 64]);
+        float x0[R / NW], x1[R / NW], cs[R / NW], sn[R / NW];
+#pragma unroll
+        for (int u = 0; u < R / NW; u++) {
+            const int row = wave + NW * u, ti = min(i0 + (row >> 1), nt - 1);
+            const float *src = qkv + (size_t)ti * QKV_LD + (size_t)(g * GRP + (row & 1)) * HD;
+            x0[u] = src[lane];
+            x1[u] = src[lane + 64];
+            cs[u] = rcos[(size_t)(pos0 + ti) * (HD / 2) + lane];
+            sn[u] = rsin[(size_t)(pos0 + ti) * (HD / 2) + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < R / NW; u++) {
+            const int row = wave + NW * u;
+            const float ss = wave_sum(sumsq2(x0[u], x1[u]));
+            const float sc = 1.0f / sqrtf(ss / (float)HD + eps);
+            float o0, o1;
+            rope_pair((x0[u] * sc) * w0, (x1[u] * sc) * w1, cs[u], sn[u], o0, o1);
+            sq[row][lane] = (row >> 1) < nq ? o0 : 0.0f;
+            sq[row][lane + 64] = (row >> 1) < nq ? o1 : 0.0f;
+        }
     }
     __syncthreads();
 
-    // scores: thread t loads key t once for all R rows
-    const f32x4 *kbase = reinterpret_cast<const f32x4 *>(kc) + (size_t)g * (HD / 4) * max_seq;
-    for (int t = tid; t < ctxmax; t += NTH) {
-        f32x4 kv[HD / 4];
+    float m[MT], l[MT];
+    f32x4 o[MT][8];
 #pragma unroll
-        for (int d4 = 0; d4 < HD / 4; d4++) kv[d4] = kbase[(size_t)d4 * max_seq + t];
+    for (int mt = 0; mt < MT; mt++) {
+        m[mt] = -INFINITY;
+        l[mt] = 0.0f;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            float sr = 0.0f;
+        for (int dt = 0; dt < 8; dt++) o[mt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (; kt < nkt; kt += kstep) {
 #pragma unroll
-            for (int d4 = 0; d4 < HD / 4; d4++) {
-                const f32x4 q = reinterpret_cast<const f32x4 *>(sq + r * HD)[d4];
-                sr = fmaf(q.x, kv[d4].x, sr); sr = fmaf(q.y, kv[d4].y, sr);
-                sr = fmaf(q.z, kv[d4].z, sr); sr = fmaf(q.w, kv[d4].w, sr);
+        for (int r = 0; r < 4; r++) {
+            const int t = 16 * kt + 4 * h + r;
+            const uint32_t off = t < ctx ? (uint32_t)((t * HD + 8 * c) * 4) : BUF_OOB;
+            vv[r][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0));
+            vv[r][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, off + 16, 0, 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // two chains per row tile, even and odd steps
+        f32x4 s0[MT], s1[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) s0[mt] = s1[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 8; s += 2) {
+            f32x4 q0[MT], q1[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                q0[mt] = *reinterpret_cast<const f32x4 *>(&sq[16 * mt + c][16 * s + 4 * h]);
+                q1[mt] = *reinterpret_cast<const f32x4 *>(&sq[16 * mt + c][16 * s + 16 + 4 * h]);
             }
-            p[r * ldp + t] = t <= pos0 + i0 + r / GRP ? sr * scale : -INFINITY;
-        }
-    }
-    __syncthreads();
-
-    // softmax per row
-    float mr[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) mr[r] = -INFINITY;
-    for (int t = tid; t < ctxmax; t += NTH)
+            for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int r = 0; r < R; r++) mr[r] = fmaxf(mr[r], p[r * ldp + t]);
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        mr[r] = wave_max(mr[r]);
-        if (lane == 0) sred[r * 4 + wave] = mr[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        mr[r] = fmaxf(fmaxf(sred[r * 4 + 0], sred[r * 4 + 1]), fmaxf(sred[r * 4 + 2], sred[r * 4 + 3]));
-    __syncthreads();
-    float er[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) er[r] = 0.0f;
-    for (int t = tid; t < ctxmax; t += NTH)
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const float av = expf(p[r * ldp + t] - mr[r]);
-            p[r * ldp + t] = av;
-            er[r] += av;
-        }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        er[r] = wave_sum(er[r]);
-        if (lane == 0) sred[r * 4 + wave] = er[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < R; r++) er[r] = (sred[r * 4 + 0] + sred[r * 4 + 1]) + (sred[r * 4 + 2] + sred[r * 4 + 3]);
-    for (int t = tid; t < ctxmax; t += NTH)
-#pragma unroll
-        for (int r = 0; r < R; r++) p[r * ldp + t] = p[r * ldp + t] / er[r];
-    __syncthreads();
-
-    // out_r[d] = sum_t p[r][t] v_t[d]: wave w takes t = w, w+4, ...; lane l
-    // owns d = 2l, 2l+1 of every row; each V row serves all R rows.  Passes
-    // of 16, then 8, 4 and 1 rows in flight per lane (each pass one L2 round
-    // trip; measured on MI355X against one 8-row pass and the 1-row tail:
-    // 64 x 2014-token batch prefill 2.71 -> 2.60 s), always adding in
-    // ascending t
-    f32x2 o[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) o[r] = f32x2{0.f, 0.f};
-    const f32x2 *vcache = reinterpret_cast<const f32x2 *>(vc + (size_t)g * max_seq * HD) + lane;
-    int t = wave;
-    auto vpass = [&](auto UC) {
-        constexpr int U = decltype(UC)::value;
-        for (; t + 4 * (U - 1) < ctxmax; t += 4 * U) {
-            f32x2 v[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) v[u] = vcache[(size_t)(t + 4 * u) * (HD / 2)];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const float pw = p[r * ldp + t + 4 * u];
-                    o[r].x = mul_add(pw, v[u].x, o[r].x);
-                    o[r].y = mul_add(pw, v[u].y, o[r].y);
+                for (int mt = 0; mt < MT; mt++) {
+                    s0[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[s][j], q0[mt][j], s0[mt], 0, 0, 0);
+                    s1[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[s + 1][j], q1[mt][j], s1[mt], 0, 0, 0);
                 }
         }
-    };
-    vpass(std::integral_constant<int, 16>{});
-    vpass(std::integral_constant<int, 8>{});
-    vpass(std::integral_constant<int, 4>{});
-    vpass(std::integral_constant<int, 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(kt + kstep);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 pr[MT];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        red[(wave * R + r) * HD + 2 * lane] = o[r].x;
-        red[(wave * R + r) * HD + 2 * lane + 1] = o[r].y;
+        for (int mt = 0; mt < MT; mt++) {
+            const int prow = pos0 + i0 + 8 * mt + (c >> 1);          // this row's own position
+            f32x4 s = (s0[mt] + s1[mt]) * ATT_SCALE;
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[r] = 16 * kt + 4 * h + r <= prow ? s[r] : -INFINITY;
+            float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+            f32x2 p = swap16(mx);
+            p = swap32(fmaxf(p.x, p.y));
+            const float mn = fmaxf(m[mt], fmaxf(p.x, p.y));
+            const float mu = mn == -INFINITY ? 0.0f : mn;            // no position of this row yet
+#pragma unroll
+            for (int r = 0; r < 4; r++) pr[mt][r] = expf(s[r] - mu);
+            const float corr = expf(m[mt] - mu);
+            l[mt] = fmaf(l[mt], corr, (pr[mt][0] + pr[mt][1]) + (pr[mt][2] + pr[mt][3]));
+            m[mt] = mn;
+            if (__any(corr != 1.0f)) {
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) o[mt][dt] *= corr;
+            }
+        }
+        bool odd = false;
+        if (16 * kt + 15 > pos0 + i0) {                              // uniform: some row does not see all 16
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) odd |= not_finite(vv[r][e >> 2][e & 3]);
+        }
+        if (!__any(odd)) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+                        o[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][dt >> 2][dt & 3], pr[mt][r], o[mt][dt], 0, 0, 0);
+        } else {
+            // the first position of the tile with such an entry: rows that
+            // see it take every V as it is, the others none that is not finite
+            int tmin = 0x7FFFFFFF;
+#pragma unroll
+            for (int r = 3; r >= 0; r--) {
+                bool b = false;
+#pragma unroll
+                for (int e = 0; e < 8; e++) b |= not_finite(vv[r][e >> 2][e & 3]);
+                if (b) tmin = 16 * kt + 4 * h + r;
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) tmin = min(tmin, __shfl_xor(tmin, d));
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) {
+                    const float v = vv[r][dt >> 2][dt & 3], vz = not_finite(v) ? 0.0f : v;
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        const f32x4 a = __builtin_amdgcn_mfma_f32_16x16x4f32(v, pr[mt][r], o[mt][dt], 0, 0, 0);
+                        const f32x4 z = __builtin_amdgcn_mfma_f32_16x16x4f32(vz, pr[mt][r], o[mt][dt], 0, 0, 0);
+                        o[mt][dt] = tmin <= pos0 + i0 + 8 * mt + (c >> 1) ? a : z;
+                    }
+                }
+        }
+    }
+    __syncthreads();                                     // the query rows are read
+
+    // this wave's partials -> LDS: row 16 mt + c, dims 32 h + 8 r + dt
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        f32x2 p = swap16(l[mt]);
+        p = swap32(p.x + p.y);
+        if (h == 0) {
+            sm[wave][16 * mt + c] = m[mt];
+            sl[wave][16 * mt + c] = p.x + p.y;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int d4 = 0; d4 < 2; d4++)
+                *reinterpret_cast<f32x4 *>(&so[wave][16 * mt + c][32 * h + 8 * r + 4 * d4]) =
+                    f32x4{o[mt][4 * d4][r], o[mt][4 * d4 + 1][r], o[mt][4 * d4 + 2][r], o[mt][4 * d4 + 3][r]};
     }
     __syncthreads();
-    for (int e = tid; e < nq * GRP * HD; e += NTH) {
-        const int r = e / HD, d = e % HD;
-        const float sacc = (red[(0 * R + r) * HD + d] + red[(1 * R + r) * HD + d]) +
-                           (red[(2 * R + r) * HD + d] + red[(3 * R + r) * HD + d]);
-        out[(size_t)(i0 + r / GRP) * (NKV * GRP * HD) + (size_t)(g * GRP + r % GRP) * HD + d] = sacc;
+    for (int e = tid; e < 2 * nq * (HD / 4); e += WAVE * NW) {
+        const int row = e / (HD / 4), d4 = e % (HD / 4);
+        float M = sm[0][row];
+#pragma unroll
+        for (int w = 1; w < NW; w++) M = fmaxf(M, sm[w][row]);
+        float L = 0.0f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float mw = sm[w][row];
+            const float wt = mw == -INFINITY ? 0.0f : expf(mw - M);   // -inf: a wave without positions of this row
+            L = fmaf(wt, sl[w][row], L);
+            acc += wt * *reinterpret_cast<const f32x4 *>(&so[w][row][4 * d4]);
+        }
+        const size_t orow = (size_t)(i0 + (row >> 1)) * (NKV * GRP) + g * GRP + (row & 1);   // [token][head]
+        if (gridDim.y == 1) {
+            reinterpret_cast<f32x4 *>(out + orow * HD)[d4] = acc / L;
+        } else {
+            float *pp = part + ((size_t)blockIdx.y * nt * (NKV * GRP) + orow) * ATT_LD;
+            reinterpret_cast<f32x4 *>(pp)[d4] = acc;
+            if (d4 == 0) { pp[HD] = M; pp[HD + 1] = L; }
+        }
     }
+}
+
+// the key splits' partials part[ks][token][head][ATT_LD] (sums, max at HD,
+// weight at HD + 1) merged into out[token][head][HD].  One block of 128
+// threads per 4 (token, head) rows, a thread per 4 dims.
+__global__ __launch_bounds__(128) void k_attn_chunk_merge(float *__restrict__ out, const float *__restrict__ part,
+                                                          int rows, int ks) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 5), d4 = threadIdx.x & 31;
+    if (row >= rows) return;
+    float m[ATT_KS], l[ATT_KS];
+    f32x4 v[ATT_KS];
+#pragma unroll
+    for (int s = 0; s < ATT_KS; s++) {
+        const float *pp = part + ((size_t)min(s, ks - 1) * rows + row) * ATT_LD;
+        v[s] = reinterpret_cast<const f32x4 *>(pp)[d4];
+        m[s] = s < ks ? pp[HD] : -INFINITY;
+        l[s] = pp[HD + 1];
+    }
+    float M = m[0];
+#pragma unroll
+    for (int s = 1; s < ATT_KS; s++) M = fmaxf(M, m[s]);
+    float L = 0.0f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < ATT_KS; s++)
+        if (m[s] != -INFINITY) {
+            const float wt = expf(m[s] - M);
+            L = fmaf(wt, l[s], L);
+            acc += wt * v[s];
+        }
+    reinterpret_cast<f32x4 *>(out + (size_t)row * HD)[d4] = acc / L;
 }
 
 // ---------------------------------------------------------------------------
@@ -695,11 +819,6 @@ __global__ void k_zero_i32(int *p, int n) {
 // ---------------------------------------------------------------------------
 static inline hipStream_t stream() { return (hipStream_t)qh_stream(); }
 
-extern "C" size_t qm_attention_lds_bytes(int qt, int ldp) {
-    const size_t r = (size_t)qt * GRP;
-    return sizeof(float) * (r * HD + 4 * r * HD + 4 * r + r * (size_t)ldp);
-}
-
 extern "C" int qm_rows_norm(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
                             const uint16_t *nw, float *xb, int nt, int K, float eps) {
     return qm_rows_norm_split(x, r, emb, tok, emb_rows, nw, xb, nt, K, eps, nullptr, 0);
@@ -719,46 +838,36 @@ extern "C" int qm_rows_norm_split(float *x, const float *r, const uint16_t *emb,
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 
-// tokens per block of the chunk attention: two while their scores fit in
-// 64 KB (contexts up to ~3,440), else one.  Measured prefill of 128 / 512 /
-// 1024 / 2048 tokens: 1.92 / 8.2 / 18.5 / 45.1 ms with two, 2.00 / 9.0 /
-// 21.4 / 56.3 with one, 2.15 / 9.7 / 23.3 / 52.2 with four (fewer blocks
-// than CUs at short contexts)
-static int attention_qt(int ldp) {
-    return qm_attention_lds_bytes(2, ldp) <= 65536 ? 2 : 1;
-}
-
-extern "C" int qm_attention(float *qkv, float *out, float *kc, float *vc, const uint16_t *qn,
+// The chunk attention's launch: 16-token blocks (each K and V load feeding two
+// row tiles) of four waves once they fill the CUs, 8-token blocks of eight
+// waves below; the context split over blocks while the grid leaves CUs idle
+// and every wave would walk at least ATT_SPLIT_TILES key tiles.
+#define ATT_SPLIT_TILES 4
+extern "C" int qm_attention(const float *qkv, float *out, float *part, float *kc, float *vc, const uint16_t *qn,
                             const uint16_t *kn, const float *rcos, const float *rsin, const int *pos_d,
                             int nt, int max_seq, int ctx_bound, float eps) {
     if (!stream()) return QH_ESTATE;
-    if (!qkv || !out || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
-    if (nt <= 0 || max_seq <= 0 || nt > QM_MAX_CHUNK || max_seq > QM_MAX_SEQ) return QH_EINVAL;
+    if (!qkv || !out || !part || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
+    if (nt <= 0 || max_seq <= 0 || nt > max_seq || max_seq > QM_MAX_SEQ) return QH_EINVAL;
     if (ctx_bound < nt || ctx_bound > max_seq) return QH_EINVAL;
-    static int attr_dev = -1;                  // the attribute is held per device
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess) return QH_ELAUNCH;
-    if (attr_dev != dev) {
-        // one token per block at the longest context needs more than the default 64 KB
-        if (hipFuncSetAttribute((const void *)k_attention<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)qm_attention_lds_bytes(1, QM_MAX_SEQ)) != hipSuccess)
-            return QH_ELAUNCH;
-        attr_dev = dev;
-    }
-    // 1 / sqrt(head_dim), the constant of qwen3.c:311
-    const float scale = 0.08838834764831845f;
-    hipLaunchKernelGGL(k_qk_rope_cache, dim3(nt, (NKV * GRP + NKV) / 4), dim3(NTH), 0, stream(), qkv, kc, vc,
-                       qn, kn, rcos, rsin, pos_d, max_seq, eps);
+    hipLaunchKernelGGL(k_rope_cache, dim3(nt, NKV / 4), dim3(NTH), 0, stream(), qkv, kc, vc, kn, rcos, rsin,
+                       pos_d, max_seq, eps);
     if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
-    const int qt = attention_qt(ctx_bound);
-    const size_t lds = qm_attention_lds_bytes(qt, ctx_bound);
-    const dim3 grid((unsigned)(((nt + qt - 1) / qt) * NKV));
-    if (qt == 2)
-        hipLaunchKernelGGL(k_attention<2>, grid, dim3(NTH), lds, stream(), qkv, out, kc, vc, pos_d, nt, max_seq,
-                           ctx_bound, scale);
-    else
-        hipLaunchKernelGGL(k_attention<1>, grid, dim3(NTH), lds, stream(), qkv, out, kc, vc, pos_d, nt, max_seq,
-                           ctx_bound, scale);
+    const int tiles = (ctx_bound + 15) / 16;
+    if ((nt + 15) / 16 * NKV >= 256) {
+        hipLaunchKernelGGL((k_attn_chunk<2, 4>), dim3((nt + 15) / 16 * NKV), dim3(4 * WAVE), 0, stream(), qkv, out,
+                           part, kc, vc, qn, rcos, rsin, pos_d, nt, max_seq, eps);
+        return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
+    }
+    const int blocks = (nt + 7) / 8 * NKV;
+    int ks = 1;
+    while (ks < ATT_KS && nt <= QM_ATT_KS_ROWS && 2 * ks * blocks <= 256 && tiles >= 8 * ks * ATT_SPLIT_TILES) ks *= 2;
+    hipLaunchKernelGGL((k_attn_chunk<1, 8>), dim3(blocks, ks), dim3(8 * WAVE), 0, stream(), qkv, out, part, kc, vc,
+                       qn, rcos, rsin, pos_d, nt, max_seq, eps);
+    if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
+    if (ks > 1)
+        hipLaunchKernelGGL(k_attn_chunk_merge, dim3(nt * (NKV * GRP) / 4), dim3(128), 0, stream(), out, part,
+                           nt * NKV * GRP, ks);
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 

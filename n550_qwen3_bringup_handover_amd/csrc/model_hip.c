@@ -51,6 +51,7 @@ struct qwen3_hip_model {
     float *rcos, *rsin;                /* [max_seq][64] */
     float *x, *x0, *x1, *xb, *qkv, *att, *ob, *hb, *dn, *logits;
     float *apart;                      /* decode attention partials [QM_ATT_PART_FLOATS] */
+    float *cpart;                      /* chunk attention partials [QM_ATT_CHUNK_PART_FLOATS] */
     int *tok_in;                       /* [QM_MAX_CHUNK] */
     int *state;                        /* [0] token, [1] position, [2] step */
     int *out_tok;                      /* [max_seq + 1] */
@@ -134,7 +135,7 @@ void qwen3_hip_model_close(qwen3_hip_model *m) {
     detach_batches(m);
     if (m->graph_id >= 0) (void)qh_graph_destroy(m->graph_id);
     void *bufs[] = {m->wbuf, m->kc, m->vc, m->rcos, m->rsin, m->x, m->x0, m->x1, m->xb, m->qkv,
-                    m->att, m->ob, m->hb, m->dn, m->logits, m->apart, m->tok_in, m->state, m->out_tok};
+                    m->att, m->ob, m->hb, m->dn, m->logits, m->apart, m->cpart, m->tok_in, m->state, m->out_tok};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++) (void)qh_free(bufs[i]);
     free(m->dump_host);
     free(m);
@@ -188,6 +189,7 @@ int qwen3_hip_model_open(qwen3_hip_model **out, const void *blob, size_t size, i
     DEV(m->dn, B * H * 4);
     DEV(m->logits, (size_t)V * 4);
     DEV(m->apart, (size_t)QM_ATT_PART_FLOATS * 4);
+    DEV(m->cpart, QM_ATT_CHUNK_PART_FLOATS * 4);
     DEV(m->tok_in, B * sizeof(int));
     DEV(m->state, 4 * sizeof(int));
     DEV(m->out_tok, ((size_t)max_seq + 1) * sizeof(int));
@@ -368,7 +370,7 @@ static int run_chunk(qwen3_hip_model *m, const kv_t *kv, int nt, int pos0, int w
         DUMP(l, "q_proj_out", m->qkv, QKV_N, 0, QW3M_Q_DIM);
         DUMP(l, "k_proj_out", m->qkv, QKV_N, QW3M_Q_DIM, QW3M_KV_DIM);
         DUMP(l, "v_proj_out", m->qkv, QKV_N, QW3M_Q_DIM + QW3M_KV_DIM, QW3M_KV_DIM);
-        if (!rc) rc = qm_attention(m->qkv, m->att, kv->kc + l * kv->layer_stride,
+        if (!rc) rc = qm_attention(m->qkv, m->att, m->cpart, kv->kc + l * kv->layer_stride,
                                    kv->vc + l * kv->layer_stride, L->qn, L->kn, m->rcos, m->rsin,
                                    m->state + 1, nt, kv->max_seq, pos0 + nt, eps);
         DUMP(l, "attn_out", m->att, QW3M_Q_DIM, 0, QW3M_Q_DIM);

@@ -13,7 +13,7 @@ extern "C" {
 #endif
 
 #define QM_MAX_CHUNK 128     /* tokens per forward call (QWEN3_MAX_BATCH, qwen3.h:145) */
-#define QM_MAX_SEQ 8192      /* positions; the attention kernels keep 2 x max_seq scores in LDS */
+#define QM_MAX_SEQ 8192      /* positions */
 
 /* x[row] = emb[tok[row]] (emb set) or x[row] += r[row] (r set);
  * xb[row] = rmsnorm(x[row]) * nw;  nt rows of K floats */
@@ -26,16 +26,18 @@ int qm_rows_norm_split(float *x_d, const float *r_d, const uint16_t *emb_d, cons
                        int ks);
 
 /* QK-norm + RoPE + KV-cache write, then causal GQA attention, for nt tokens
- * at positions *pos_d .. *pos_d + nt - 1 of one layer (two launches); the
- * q part of qkv is left normalised and roped.  ctx_bound (host-known,
- * nt .. max_seq) must be >= *pos_d + nt: it sizes the scores in LDS (tokens
- * whose context exceeds it are skipped) */
-int qm_attention(float *qkv_d, float *out_d, float *kc_d, float *vc_d, const uint16_t *qn_d,
-                 const uint16_t *kn_d, const float *rcos_d, const float *rsin_d, const int *pos_d,
-                 int nt, int max_seq, int ctx_bound, float eps);
-/* dynamic LDS of the chunk attention with qt tokens per block and score
- * rows of ldp floats */
-size_t qm_attention_lds_bytes(int qt, int ldp);
+ * at positions *pos_d .. *pos_d + nt - 1 of one layer (two launches, three
+ * where a short chunk's context is split over blocks).  ctx_bound (host-known,
+ * nt .. max_seq) is *pos_d + nt: it picks the split.  part_d:
+ * QM_ATT_CHUNK_PART_FLOATS of scratch for the splits' partials, each
+ * QM_ATT_PART floats per token and head, QM_ATT_KS splits of at most
+ * QM_ATT_KS_ROWS tokens */
+#define QM_ATT_KS 8
+#define QM_ATT_KS_ROWS 128
+#define QM_ATT_CHUNK_PART_FLOATS ((size_t)QM_ATT_KS * QM_ATT_KS_ROWS * 16 * QH_ATT_PART)
+int qm_attention(const float *qkv_d, float *out_d, float *part_d, float *kc_d, float *vc_d,
+                 const uint16_t *qn_d, const uint16_t *kn_d, const float *rcos_d, const float *rsin_d,
+                 const int *pos_d, int nt, int max_seq, int ctx_bound, float eps);
 
 /* decode attention split into QM_ATT_SPLITS position ranges per kv head:
  * writes softmax partials (m, l, o[128] per head and range, QM_ATT_PART
