@@ -52,7 +52,7 @@ struct qwen3_hip_model {
     float *x, *x0, *x1, *xb, *qkv, *att, *ob, *hb, *dn, *logits;
     float *apart;                      /* decode attention partials [QM_ATT_PART_FLOATS] */
     float *cpart;                      /* chunk attention partials [QM_ATT_CHUNK_PART_FLOATS] */
-    int *tok_in;                       /* [QM_MAX_CHUNK] */
+    int *tok_in;                       /* [prefill_rows(max_seq)] */
     int *state;                        /* [0] token, [1] position, [2] step */
     int *out_tok;                      /* [max_seq + 1] */
     int use_graph;
@@ -87,6 +87,14 @@ int qwen3_hip_qw3m_check(const void *blob, size_t size) { return qw3m_parse(blob
 /* ---- open / close ------------------------------------------------------------ */
 
 static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+/* rows of the chunk buffers: the tokens one pass of the layers takes at most
+ * (forward() takes up to QM_MAX_CHUNK per call, which a smaller cache does
+ * not lower) */
+static int prefill_rows(int max_seq) {
+    const int n = max_seq < QM_PREFILL_ROWS ? max_seq : QM_PREFILL_ROWS;
+    return n > QM_MAX_CHUNK ? n : QM_MAX_CHUNK;
+}
 
 /* bytes of each device tensor, in allocation order */
 static size_t dev_weight_bytes(void) {
@@ -177,7 +185,7 @@ int qwen3_hip_model_open(qwen3_hip_model **out, const void *blob, size_t size, i
     const size_t rope_bytes = (size_t)max_seq * (QW3M_HEAD_DIM / 2) * sizeof(float);
     DEV(m->rcos, rope_bytes);
     DEV(m->rsin, rope_bytes);
-    const size_t B = QM_MAX_CHUNK;
+    const size_t B = (size_t)prefill_rows(max_seq);
     DEV(m->x, B * H * 4);
     DEV(m->x0, H * 4);
     DEV(m->x1, H * 4);
@@ -458,6 +466,22 @@ static int load_chunk(qwen3_hip_model *m, const int *tokens, int nt, int pos0) {
     return rc;
 }
 
+/* a whole prompt at positions 0 .. n - 1 into the sequence whose cache is kv,
+ * in equal passes of at most prefill_rows tokens (QM_MAX_CHUNK while a dump
+ * callback wants each pass's tensors); logits of the last token.  *last: the
+ * tokens of the last pass. */
+static int prefill(qwen3_hip_model *m, const kv_t *kv, const int *prompt, int n, int *last) {
+    const int most = m->dump ? QM_MAX_CHUNK : prefill_rows(m->max_seq);
+    const int passes = (n + most - 1) / most, each = (n + passes - 1) / passes;
+    int rc = QWEN3_HIP_OK;
+    for (int p0 = 0; p0 < n && !rc; p0 += each) {
+        *last = n - p0 < each ? n - p0 : each;
+        rc = load_chunk(m, prompt + p0, *last, p0);
+        if (!rc) rc = run_chunk(m, kv, *last, p0, p0 + *last == n);
+    }
+    return rc;
+}
+
 int qwen3_hip_model_forward(qwen3_hip_model *m, const int *tokens, int n_token, int pos0) {
     if (!m || !tokens) return QWEN3_HIP_EINVAL;
     if (n_token < 1 || n_token > QM_MAX_CHUNK || pos0 < 0 || pos0 + n_token > m->max_seq)
@@ -496,11 +520,7 @@ int qwen3_hip_model_generate(qwen3_hip_model *m, const int *prompt, int n_prompt
     const kv_t kv = model_kv(m);
     const double t0 = now_ms();
     int nt = 0;
-    for (int p0 = 0; p0 < n_prompt && !rc; p0 += QM_MAX_CHUNK) {
-        nt = n_prompt - p0 < QM_MAX_CHUNK ? n_prompt - p0 : QM_MAX_CHUNK;
-        rc = load_chunk(m, prompt + p0, nt, p0);
-        if (!rc) rc = run_chunk(m, &kv, nt, p0, p0 + nt == n_prompt);
-    }
+    rc = prefill(m, &kv, prompt, n_prompt, &nt);
     /* first token; state[1] = pos0 of the last chunk + nt = n_prompt */
     if (!rc) rc = qm_set_i32(m->state + 2, 0);
     if (!rc) rc = qh_argmax_step(m->state, m->out_tok, m->state + 2, m->max_seq + 1, m->state + 1, nt,
@@ -663,11 +683,8 @@ int qwen3_hip_batch_prefill(qwen3_hip_batch *b, int seq, const int *prompt, int 
                      (size_t)b->n_seq * b->kv_seq, b->max_ctx};
     b->h_next[seq] = -1;
     m->have_logits = 0;             /* the model's logits buffer is reused below */
-    for (int p0 = 0; p0 < n_prompt && !rc; p0 += QM_MAX_CHUNK) {
-        const int nt = n_prompt - p0 < QM_MAX_CHUNK ? n_prompt - p0 : QM_MAX_CHUNK;
-        rc = load_chunk(m, prompt + p0, nt, p0);
-        if (!rc) rc = run_chunk(m, &kv, nt, p0, p0 + nt == n_prompt);
-    }
+    int nt = 0;
+    rc = prefill(m, &kv, prompt, n_prompt, &nt);
     /* first token: out[seq][0] at pos - plen + 1 = 0, then pos = n_prompt */
     if (!rc) rc = qm_set_i32(b->pos + seq, n_prompt - 1);
     if (!rc) rc = qm_set_i32(b->plen + seq, n_prompt);

@@ -13,6 +13,7 @@ extern "C" {
 #endif
 
 #define QM_MAX_CHUNK 128     /* tokens per forward call (QWEN3_MAX_BATCH, qwen3.h:145) */
+#define QM_PREFILL_ROWS 2048 /* tokens per pass of a prompt: the chunk buffers are 52 KB a token */
 #define QM_MAX_SEQ 8192      /* positions */
 
 /* x[row] = emb[tok[row]] (emb set) or x[row] += r[row] (r set);
