@@ -810,6 +810,16 @@ __global__ void k_set_i32(int *p, int v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) p[0] = v;
 }
 
+struct Tokens {
+    int t[QM_MAX_CHUNK];
+};
+__global__ __launch_bounds__(QM_MAX_CHUNK) void k_set_tokens(int *__restrict__ tok, Tokens v, int n,
+                                                             int *__restrict__ pos, int pos0) {
+    const int i = threadIdx.x;
+    if (i < n) tok[i] = v.t[i];
+    if (i == 0) *pos = pos0;
+}
+
 __global__ void k_zero_i32(int *p, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
@@ -915,6 +925,15 @@ extern "C" int qm_zero_i32(int *p, int n) {
     if (n == 0) return QH_OK;
     hipLaunchKernelGGL(k_zero_i32, dim3((n + NTH - 1) / NTH < 1024 ? (n + NTH - 1) / NTH : 1024), dim3(NTH), 0,
                        stream(), p, n);
+    return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
+}
+
+extern "C" int qm_set_tokens(int *tok, const int *tokens, int n, int *pos, int pos0) {
+    if (!stream()) return QH_ESTATE;
+    if (!tok || !tokens || !pos || n <= 0 || n > QM_MAX_CHUNK) return QH_EINVAL;
+    Tokens v = {};
+    for (int i = 0; i < n; i++) v.t[i] = tokens[i];
+    hipLaunchKernelGGL(k_set_tokens, dim3(1), dim3(QM_MAX_CHUNK), 0, stream(), tok, v, n, pos, pos0);
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 

@@ -89,6 +89,9 @@ int qm_decode_layers_persist(const uint16_t *const *w, int layers, const uint16_
                              const float *rsin, int max_seq, float eps, float *x_out, float *dn_out);
 int qm_persist_errors(unsigned *flags);
 
+/* tok[0 .. n) = the host's tokens (n <= QM_MAX_CHUNK) and *pos = pos0, both
+ * passed as kernel arguments: the caller's buffer is read before the return */
+int qm_set_tokens(int *tok_d, const int *tokens, int n, int *pos_d, int pos0);
 /* *p = v, as a kernel (safe inside stream capture) */
 int qm_set_i32(int *p_d, int v);
 /* p[0..n) = 0, as a kernel */
