@@ -281,7 +281,11 @@ enum {
     // M <= 16, K = 1024, 2048 or 3072: 16-column blocks, K split over the
     // block's waves, v_mfma_f32_16x16x32_bf16 (not gated)
     PLAN_M16 = 27,
-    PLAN_COUNT = 28
+    // large-tile kernel for K % 64 != 0 or operands that are not 16-byte
+    // aligned (not gated)
+    PLAN_R64x64 = 28,          // three register sets
+    PLAN_R128x128 = 29,
+    PLAN_COUNT = 30
 };
 static const char *k_plan_names[PLAN_COUNT] = {
     "auto", "gemv", "mfma128x128", "mfma64x128", "mfma64x64", "mfma32x128", "mfma16x64", "mfma64x64-scalar",
@@ -289,13 +293,19 @@ static const char *k_plan_names[PLAN_COUNT] = {
     "xl128x128", "xl256x256", "xl64x128",
     "xb256x256k32", "xb128x128", "xb256x256s1",
     "stream", "stream-ks1", "stream-ks2", "stream-ks4", "stream-ks8", "skinny", "narrow", "wide",
-    "gemv16", "xl64x64s3", "m16"};
+    "gemv16", "xl64x64s3", "m16", "rag64x64", "rag128x128"};
 static inline bool is_pipe_plan(int p) { return p >= PLAN_P32x64k128s4 && p <= PLAN_P64x64k64s3; }
 static inline bool is_xl_plan(int p) {
     return (p >= PLAN_X128x128 && p <= PLAN_XB256x256s1) || p == PLAN_X64x64s3;
 }
 static inline bool is_xb_plan(int p) { return p >= PLAN_XB256x256k32 && p <= PLAN_XB256x256s1; }
 static inline bool is_stream_plan(int p) { return p >= PLAN_STREAM && p <= PLAN_STREAM_KS8; }
+static inline bool is_rag_plan(int p) { return p == PLAN_R64x64 || p == PLAN_R128x128; }
+// the ragged large tiles' limits: byte offsets below 2 GiB (their
+// out-of-range marker)
+static inline bool rag_fits(int M, int K, int N) {
+    return K > 0 && (size_t)M * K * 4 < (1ull << 31) && (size_t)N * K * 2 < (1ull << 31);
+}
 static inline bool is_narrow_plan(int p) { return p == PLAN_NARROW; }
 static inline int stream_mt(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
 // the stream kernel's limits: M <= 64, whole 256-deep block slices, byte
@@ -371,8 +381,28 @@ static int choose_bf16a_plan(int M, int K, int N, int gated) {
     return PLAN_XB128x128;
 }
 
+// K % 64 != 0, or (vec false) K % 8 != 0 or operands not 16-byte aligned: the
+// large-tile kernel with a ragged last stage, 64 x 64 tiles while they make at
+// most two rounds, else 128 x 128 (measured on MI355X, graph-replayed, K % 8
+// == 0: 333 x 1000 x 2501 15.8 -> 9.4 us against the register-staged 64 x 64
+// tiles, 128 x 1000 x 1000 15.5 -> 9.3, 24 x 1896 x 1500 27.6 -> 11.4, 700 x
+// 1992 x 4000 36.7 -> 27.9 on 128 x 128 (43.0 on 64 x 64); K odd, against
+// element-wise loads: 500 x 1999 x 4000 142 -> 32.8, 16 x 1001 x 3000 43.6 ->
+// 9.2, 3 x 100 x 100 5.2 -> 4.1).  Not where K makes one stage of edge loads
+// (K < 64), nor aligned with more than one round of 128 x 128 tiles, where the
+// register-staged tiles stay ahead (2000 x 1000 x 3000 30.3 against 36.0 us).
+static int choose_rag_plan(int M, int K, int N, int gated, bool vec) {
+    if (gated || K < 64 || !rag_fits(M, K, N)) return PLAN_AUTO;
+    const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (t64 <= 2 * g_cus) return PLAN_R64x64;
+    return (t128 <= g_cus || !vec) ? PLAN_R128x128 : PLAN_AUTO;
+}
+
 static int choose_plan(int M, int K, int N, int gated, bool vec) {
-    if (!vec) return PLAN_SCALAR64;
+    if (!vec) {
+        const int p = choose_rag_plan(M, K, N, gated, false);
+        return p != PLAN_AUTO ? p : PLAN_SCALAR64;
+    }
     // 2 <= M <= 16 (config 1's gate_proj, small decode batches): the 16-row
     // kernel, 16 or 32 columns per block and K split over its waves, where a
     // sweep of M 2..16 x K 1024..3072 x N 1024..16384 measured it fastest
@@ -525,6 +555,10 @@ static int choose_plan(int M, int K, int N, int gated, bool vec) {
         }
         if (M > 128 && blocks(128, 128) >= 128)
             return (!gated && blocks(64, 128) >= 256) ? PLAN_X64x128 : PLAN_X128x128;
+    }
+    if (K % 64 != 0) {
+        const int p = choose_rag_plan(M, K, N, gated, true);
+        if (p != PLAN_AUTO) return p;
     }
     if (M <= 128 || (!gated && M <= 512)) {
         const long t = blocks(32, 64);
@@ -901,7 +935,7 @@ static int launch_xl(float *c, const void *a, const uint16_t *b, const uint16_t 
     if (tiles < 0) return QH_ETOOBIG;
     if constexpr (GATED && BM == 128 && BN == 128) {
         if (tiles <= g_cus) {
-            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 4, 1>), dim3((unsigned)tiles, 1),
+            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 4, 1, 0>), dim3((unsigned)tiles, 1),
                                dim3(XlCfg<BM, BN, BK, GATED, ABF16, SETS, 4>::NT), 0, g_stream, c, a, b, b2, M, K, N,
                                map);
             HCHECK(hipGetLastError(), QH_ELAUNCH);
@@ -910,17 +944,37 @@ static int launch_xl(float *c, const void *a, const uint16_t *b, const uint16_t 
     }
     if constexpr (BK == 64 && BM * BN <= 128 * 128 && (!GATED || BM * BN < 128 * 128)) {
         if (tiles <= g_cus) {
-            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 2>), dim3((unsigned)tiles, 1),
+            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 2, 0>), dim3((unsigned)tiles, 1),
                                dim3(XlCfg<BM, BN, BK, GATED, ABF16, SETS, 2, 2>::NT), 0, g_stream, c, a, b, b2, M, K, N,
                                map);
             HCHECK(hipGetLastError(), QH_ELAUNCH);
             return QH_OK;
         }
     }
-    hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 1>), dim3((unsigned)tiles, 1), dim3(X::NT), 0,
+    hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 1, 0>), dim3((unsigned)tiles, 1), dim3(X::NT), 0,
                        g_stream, c, a, b, b2, M, K, N, map);
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
+}
+
+// ragged large tiles, always two k groups of four waves (with one, the
+// unaligned 128 x 128 kernel spills); sizes within rag_fits
+template <int BM, int BN, int SETS, int RAG>
+static int launch_rag_t(float *c, const float *a, const uint16_t *b, int M, int K, int N) {
+    TileMap map;
+    const long tiles = make_map(map, M, N, K, BM, BN, BN);
+    if (tiles < 0) return QH_ETOOBIG;
+    hipLaunchKernelGGL((k_gemm_xl<BM, BN, 64, false, false, SETS, 2, 2, RAG>), dim3((unsigned)tiles, 1),
+                       dim3(XlCfg<BM, BN, 64, false, false, SETS, 2, 2>::NT), 0, g_stream, c, a, b, nullptr, M, K, N,
+                       map);
+    HCHECK(hipGetLastError(), QH_ELAUNCH);
+    return QH_OK;
+}
+static int launch_rag(int plan, float *c, const float *a, const uint16_t *b, int M, int K, int N) {
+    const bool vec = K % 8 == 0 && aligned16(a) && aligned16(b);
+    if (plan == PLAN_R64x64)
+        return vec ? launch_rag_t<64, 64, 3, 1>(c, a, b, M, K, N) : launch_rag_t<64, 64, 3, 2>(c, a, b, M, K, N);
+    return vec ? launch_rag_t<128, 128, 2, 1>(c, a, b, M, K, N) : launch_rag_t<128, 128, 2, 2>(c, a, b, M, K, N);
 }
 
 // fp32 -> bf16 (RNE) on the stream; n % 8 == 0, 16-byte aligned pointers
@@ -1332,6 +1386,9 @@ static int dispatch(int plan, const Ws &ws, float *c, const float *a, const uint
         case PLAN_X256x256: return launch_xl<256, 256, 32, GATED>(c, a, b, b2, M, K, N);
         case PLAN_X64x128:  return launch_xl<64, 128, 64, GATED>(c, a, b, b2, M, K, N);
         case PLAN_X64x64s3: return launch_xl<64, 64, 64, false, false, 3>(c, a, b, b2, M, K, N);   // not gated
+        case PLAN_R64x64: case PLAN_R128x128:
+            if constexpr (GATED) return QH_EINVAL;
+            else return launch_rag(plan, c, a, b, M, K, N);
         case PLAN_SKINNY: return launch_skinny<GATED>(ws, c, a, b, b2, M, K, N);
         case PLAN_NARROW:
             return launch_narrow<GATED>(ws, c, a, b, b2, M, K, N);
@@ -1358,7 +1415,8 @@ static int dispatch(int plan, const Ws &ws, float *c, const float *a, const uint
 // -QH_E* on error.
 static int resolve_plan(Ws &ws, int M, int K, int N, bool gated, bool vec, bool strict) {
     int plan = g_forced_plan ? g_forced_plan : choose_plan(M, K, N, gated, vec);
-    if (!vec) plan = PLAN_SCALAR64;   // forced plans still need vector-safe inputs
+    if (is_rag_plan(plan) && (gated || !rag_fits(M, K, N))) plan = vec ? PLAN_T64x64 : PLAN_SCALAR64;
+    if (!vec && !is_rag_plan(plan)) plan = PLAN_SCALAR64;   // forced plans still need vector-safe inputs
     if (plan == PLAN_GEMV && (M > 4 || (size_t)M * K * 4 > 64 * 1024)) plan = PLAN_T64x64;
     if (is_pipe_plan(plan) && (K % pipe_bk(plan)) != 0) plan = PLAN_T64x64;   // whole k stages
     if (plan == PLAN_X64x64s3 && gated) plan = PLAN_T64x64;   // one B block per wave tile

@@ -711,6 +711,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t xl_rsrc(const void *p, size_t 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)(uint32_t)bytes, 0x00020000);
 }
 
+// 16 bytes at an address aligned to an element only
+typedef unsigned int u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
 // ABF16: A is already bf16 (a points to uint16_t bits): it is copied into LDS
 // like B, with no conversion.
 // 64-row tiles (batched decode) are bandwidth kernels: two blocks per CU
@@ -718,7 +722,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t xl_rsrc(const void *p, size_t 
 // SETS = 1: one register set; each stage stores stage it+1 first and then
 // loads stage it+2 into the freed registers (one stage of latency cover, for
 // tiles whose two register sets would not fit).
-template <int BM, int BN, int BK, bool GATED, bool ABF16, int SETS, int WMW, int KG>
+// RAG: what K and the operands' addresses may be.  0: K % BK == 0, 16-byte
+// aligned; 1: K % 8 == 0, 16-byte aligned: the last stage's chunks past K are
+// loaded out of range (zeros); 2: any K, elements aligned to their own size
+// only: 16-byte loads at those addresses, and the last stage element by
+// element, out of range past K.  Only the last stage differs, and it is loaded
+// in the prologue or the tail, so the steady loop is the aligned kernel's.
+// RAG 1 and 2 need A and B below 2 GiB each (the out-of-range marker).
+template <int BM, int BN, int BK, bool GATED, bool ABF16, int SETS, int WMW, int KG, int RAG>
 __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) * KG == 8 ? 1 : (BM * BN <= 128 * 128 ? 2 : 1)) void k_gemm_xl(float *__restrict__ c,
                                                         const void *__restrict__ a,
                                                         const uint16_t *__restrict__ b,
@@ -740,7 +751,8 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
     tile_of(blockIdx.x, map, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * X::BNO;
-    const int nk = K / BK;
+    const int nk = RAG ? (K + BK - 1) / BK : K / BK;
+    static_assert(RAG == 0 || (!GATED && !ABF16), "ragged K: plain products of fp32 A");
 
     const __amdgpu_buffer_rsrc_t ra = xl_rsrc(a, (size_t)M * K * (ABF16 ? 2 : 4));
     const __amdgpu_buffer_rsrc_t rb = xl_rsrc(b, (size_t)N * K * 2);
@@ -799,6 +811,15 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
     auto load = [&](int step, auto SET) {
         constexpr int set = SETS == 1 ? 0 : decltype(SET)::value % SETS;
         const int ka = step * BK * (ABF16 ? 2 : 4), kb = step * BK * 2;   // scalar byte offsets
+        if constexpr (RAG == 2) {
+#pragma unroll
+            for (int i = 0; i < X::A_LOADS; i++)
+                areg[set][i] = *reinterpret_cast<const u32x4_a4 *>(reinterpret_cast<const char *>(a) + ka + aoffs[i]);
+#pragma unroll
+            for (int i = 0; i < X::B_LOADS; i++)
+                breg[set][i] = *reinterpret_cast<const u32x4_a2 *>(reinterpret_cast<const char *>(b) + kb + boffs[i]);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < X::A_LOADS; i++)
             areg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoffs[i], ka, 0);
@@ -806,6 +827,44 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
         for (int i = 0; i < X::B_LOADS; i++) {
             const bool up = GATED && i * X::B_ROWS_PER_LOAD >= X::BNO;
             breg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(up ? rb2 : rb, boffs[i], kb, 0);
+        }
+    };
+    // stage `step` where it may be the last one
+    auto load_tail = [&](int step, auto SET) {
+        if constexpr (RAG == 0) {
+            load(step, SET);
+        } else {
+            if (step + 1 < nk) {
+                load(step, SET);
+                return;
+            }
+            constexpr int set = SETS == 1 ? 0 : decltype(SET)::value % SETS;
+            const uint32_t ka = (uint32_t)step * BK * 4, kb = (uint32_t)step * BK * 2;
+            const int ac = step * BK + tid % X::A_CPR * 4, bc = step * BK + tid % CPR * 8;   // this lane's k of every load
+            if constexpr (RAG == 1) {
+#pragma unroll
+                for (int i = 0; i < X::A_LOADS; i++)
+                    areg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(ra, ac < K ? aoffs[i] + ka : BUF_OOB, 0, 0);
+#pragma unroll
+                for (int i = 0; i < X::B_LOADS; i++)
+                    breg[set][i] = __builtin_amdgcn_raw_buffer_load_b128(rb, bc < K ? boffs[i] + kb : BUF_OOB, 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < X::A_LOADS; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        areg[set][i][e] = __builtin_amdgcn_raw_buffer_load_b32(ra, ac + e < K ? aoffs[i] + ka + 4 * e : BUF_OOB, 0, 0);
+#pragma unroll
+                for (int i = 0; i < X::B_LOADS; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t lo = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                            rb, bc + 2 * e < K ? boffs[i] + kb + 4 * e : BUF_OOB, 0, 0);
+                        const uint32_t hi = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                            rb, bc + 2 * e + 1 < K ? boffs[i] + kb + 4 * e + 2 : BUF_OOB, 0, 0);
+                        breg[set][i][e] = lo | hi << 16;
+                    }
+            }
         }
     };
     // RSET: the register set that holds the stage (SETS = 3: not the slot)
@@ -872,18 +931,18 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
     // prologue: stage 0 stored, stage 1 (and with two sets stage 1 too)
     // in flight
     if constexpr (SETS == 3) {
-        load(0, IC<0>{});
-        if (nk > 1) load(1, IC<1>{});
-        if (nk > 2) load(2, IC<2>{});
+        load_tail(0, IC<0>{});
+        if (nk > 1) load_tail(1, IC<1>{});
+        if (nk > 2) load_tail(2, IC<2>{});
         store(IC<0>{}, IC<0>{});
     } else if constexpr (SETS == 2) {
-        load(0, IC<0>{});
-        if (nk > 1) load(1, IC<1>{});
+        load_tail(0, IC<0>{});
+        if (nk > 1) load_tail(1, IC<1>{});
         store(IC<0>{}, IC<0>{});
     } else {
-        load(0, IC<0>{});
+        load_tail(0, IC<0>{});
         store(IC<0>{}, IC<0>{});
-        if (nk > 1) load(1, IC<0>{});
+        if (nk > 1) load_tail(1, IC<0>{});
     }
     __syncthreads();
 
@@ -907,12 +966,12 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
     auto tail = [&](int it, auto SET) {
         constexpr int set = decltype(SET)::value;
         if constexpr (SETS == 2) {
-            if (it + 2 < nk) load(it + 2, IC<set>{});
+            if (it + 2 < nk) load_tail(it + 2, IC<set>{});
             compute(IC<set>{});
             if (it + 1 < nk) store(IC<set ^ 1>{}, IC<set ^ 1>{});
         } else {
             if (it + 1 < nk) store(IC<set ^ 1>{}, IC<0>{});
-            if (it + 2 < nk) load(it + 2, IC<0>{});
+            if (it + 2 < nk) load_tail(it + 2, IC<0>{});
             compute(IC<set>{});
         }
         __syncthreads();
@@ -930,14 +989,15 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
     };
     auto tail3 = [&](int it, auto R) {
         constexpr int r = decltype(R)::value;
-        if (it + 3 < nk) load(it + 3, IC<r % 3>{});
+        if (it + 3 < nk) load_tail(it + 3, IC<r % 3>{});
         compute(IC<r & 1>{});
         if (it + 1 < nk) store(IC<(r + 1) & 1>{}, IC<(r + 1) % 3>{});
         __syncthreads();
     };
+    constexpr int LATE = RAG ? 1 : 0;          // the last stage is never a steady load
     int it = 0;
     if constexpr (SETS == 3) {
-        for (; it + 8 < nk; it += 6) {
+        for (; it + 8 + LATE < nk; it += 6) {
             steady3(it, IC<0>{});
             steady3(it + 1, IC<1>{});
             steady3(it + 2, IC<2>{});
@@ -945,7 +1005,7 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
             steady3(it + 4, IC<4>{});
             steady3(it + 5, IC<5>{});
         }
-        // at most 8 stages left, it a multiple of 6
+        // at most 8 (9) stages left, it a multiple of 6
         tail3(it, IC<0>{});
         if (it + 1 < nk) tail3(it + 1, IC<1>{});
         if (it + 2 < nk) tail3(it + 2, IC<2>{});
@@ -954,15 +1014,21 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
         if (it + 5 < nk) tail3(it + 5, IC<5>{});
         if (it + 6 < nk) tail3(it + 6, IC<0>{});
         if (it + 7 < nk) tail3(it + 7, IC<1>{});
+        if constexpr (LATE) {
+            if (it + 8 < nk) tail3(it + 8, IC<2>{});
+        }
     } else {
-        for (; it + 3 < nk; it += 2) {
+        for (; it + 3 + LATE < nk; it += 2) {
             steady(it, IC<0>{});
             steady(it + 1, IC<1>{});
         }
-        // 1 to 3 stages left, it even
+        // 1 to 3 (4) stages left, it even
         tail(it, IC<0>{});
         if (it + 1 < nk) tail(it + 1, IC<1>{});
         if (it + 2 < nk) tail(it + 2, IC<0>{});
+        if constexpr (LATE) {
+            if (it + 3 < nk) tail(it + 3, IC<1>{});
+        }
     }
 
     // two wave groups: the second adds its sums into the first's through LDS

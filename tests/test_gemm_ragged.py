@@ -1,0 +1,60 @@
+"""GEMMs whose K is no multiple of 64 or whose operands are not 16-byte
+aligned: the large-tile kernel with a ragged last stage, against the oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from n550_qwen3_bringup_handover_amd import abi, runtime
+from tests import numerics
+
+# K: one to eleven stages of 64 (the three-set pipeline's tails), whole and
+# ragged last stages, multiples of 8 and not; M, N: one row or column, tile
+# edges and partial tiles
+SHAPES = [(1, 64, 1), (65, 65, 63), (64, 72, 128), (3, 100, 100), (130, 129, 129), (63, 191, 200), (7, 256, 65),
+          (100, 321, 70), (33, 392, 257), (129, 450, 64), (16, 513, 130), (40, 577, 66), (64, 640, 64),
+          (5, 703, 300), (128, 641, 128), (66, 1000, 90), (17, 1999, 33)]
+
+
+@pytest.mark.parametrize("M,K,N,gated,plan", [
+    (333, 1000, 2501, False, "rag64x64"), (700, 1992, 4000, False, "rag128x128"),
+    (500, 1999, 4000, False, "rag64x64"), (700, 1999, 4000, False, "rag128x128"),
+    (3, 100, 100, False, "rag64x64"), (3, 1000, 3000, False, "gemv"),
+    (16, 520, 3000, False, "gemv16"), (2000, 1000, 3000, False, "mfma128x128"),
+    (2000, 1001, 3000, False, "rag128x128"), (16, 63, 128, False, "mfma64x64-scalar"),
+    (64, 1001, 512, True, "mfma64x64-scalar"), (64, 40, 512, False, "mfma64x64"),
+    (30000, 20001, 64, False, "mfma64x64-scalar"),          # A past 2 GiB
+])
+def test_ragged_plan_rule(M, K, N, gated, plan):
+    assert abi.plan(M, K, N, gated) == plan
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", ["rag64x64", "rag128x128"])
+@pytest.mark.parametrize("shift", [0, 1], ids=["aligned", "unaligned"])
+def test_ragged_kernel(plan, shift):
+    """Operands inside NaN (0x7FC0) buffers, one element past a 16-byte
+    boundary when shifted: a value read outside the operands, or a k past K
+    that is not zero, makes outputs NaN.  Tolerances as in numerics.compare."""
+    L = runtime.init()
+    abi.force_plan(abi.PLANS[plan])
+    try:
+        for M, K, N in SHAPES:
+            print(f"{plan} shift {shift} {M}x{K}x{N}", flush=True)
+            a = oracle.f32_bf16_normal(M * K, 5200 + M + K + N, 1.0)
+            b = oracle.bf16_normal(N * K, 5201 + M + K + N, 0.02)
+            pa = np.full(M * K + 264, np.nan, np.float32)
+            pb = np.full(N * K + 264, 0x7FC0, np.uint16)
+            pa[128 + shift:128 + shift + M * K] = a
+            pb[128 + shift:128 + shift + N * K] = b
+            ad, bd = abi.DeviceBuffer.from_array(pa), abi.DeviceBuffer.from_array(pb)
+            cd = abi.DeviceBuffer.from_array(np.full(M * N + 64, np.nan, np.float32))
+            runtime.check(L.qwen3_hip_gemm_dev(ctypes.c_void_p(cd.ptr), ctypes.c_void_p(ad.ptr + 4 * (128 + shift)),
+                                               ctypes.c_void_p(bd.ptr + 2 * (128 + shift)), M, K, N), "gemm_dev")
+            assert abi.last_plan() == plan
+            c = cd.download(np.float32, M * N + 64)
+            numerics.compare(c[:M * N], a, b, M, K, N)
+            assert np.isnan(c[M * N:]).all()                # nothing written past C
+    finally:
+        abi.force_plan(0)
