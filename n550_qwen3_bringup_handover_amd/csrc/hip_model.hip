@@ -526,6 +526,8 @@ __global__ __launch_bounds__(128) void k_attn_chunk_merge(float *__restrict__ ou
 // ~2040: 172 -> 163 us per layer launch).
 __device__ __forceinline__ int attn_chunk(int ctx, int S) { return ((ctx + S - 1) / S + 7) & ~7; }
 
+// With one split (S = 1) the block holds the whole softmax and writes
+// part[seq][16 heads x 128] = o / l: the attention output itself.
 template <int S>
 __global__ __launch_bounds__(NTH) void k_attn_part(const float *__restrict__ qkv,
                                                    float *__restrict__ part,
@@ -544,7 +546,7 @@ __global__ __launch_bounds__(NTH) void k_attn_part(const float *__restrict__ qkv
     qkv += (size_t)seq * QKV_LD;
     kc += (size_t)seq * kv_seq;
     vc += (size_t)seq * kv_seq;
-    part += (size_t)seq * (8 * S * GRP * QM_ATT_PART);
+    part += (size_t)seq * (S == 1 ? NKV * GRP * HD : 8 * S * GRP * QM_ATT_PART);
     const int pos = pos_d[seq];
     if (pos < 0 || pos >= max_seq) return;      // uniform per launch
     const int ctx = pos + 1;
@@ -694,6 +696,13 @@ __global__ __launch_bounds__(NTH) void k_attn_part(const float *__restrict__ qkv
     // sum the 8 lanes of each chunk (lanes c, c+8, ..., c+56) and write
     o0 = f32x4{sum_stride8(o0.x), sum_stride8(o0.y), sum_stride8(o0.z), sum_stride8(o0.w)};
     o1 = f32x4{sum_stride8(o1.x), sum_stride8(o1.y), sum_stride8(o1.z), sum_stride8(o1.w)};
+    if constexpr (S == 1) {
+        if (lane < 8) {
+            reinterpret_cast<f32x4 *>(part + (size_t)g * GRP * HD)[vch] = o0 * (1.0f / l0);
+            reinterpret_cast<f32x4 *>(part + ((size_t)g * GRP + 1) * HD)[vch] = o1 * (1.0f / l1);
+        }
+        return;
+    }
     float *pp = part + (size_t)(g * S + sp) * GRP * QM_ATT_PART;
     if (lane < 8) {
         reinterpret_cast<f32x4 *>(pp + 4)[vch] = o0;
@@ -881,18 +890,41 @@ extern "C" int qm_attention(const float *qkv, float *out, float *part, float *kc
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 
+// n_seq sequences' decode attention in S ranges per kv head, merged into att
+template <int S>
+static int launch_attn_decode(const float *qkv, float *att, float *part, float *kc, float *vc, size_t kv_seq,
+                              const uint16_t *qn, const uint16_t *kn, const float *rcos, const float *rsin,
+                              const int *pos_d, int n_seq, int max_seq, float eps) {
+    hipLaunchKernelGGL(k_attn_part<S>, dim3(NKV * S, n_seq), dim3(NTH), 0, stream(), qkv, S == 1 ? att : part, kc, vc,
+                       qn, kn, rcos, rsin, pos_d, max_seq, kv_seq, eps, ATT_SCALE);
+    if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
+    if constexpr (S > 1) {
+        hipLaunchKernelGGL(k_attn_merge<S>, dim3(NKV, n_seq), dim3(NTH), 0, stream(), att, part);
+        if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
+    }
+    return QH_OK;
+}
+
 extern "C" int qm_attention_decode_part(const float *qkv, float *part, float *kc, float *vc, const uint16_t *qn,
                                         const uint16_t *kn, const float *rcos, const float *rsin,
                                         const int *pos_d, int max_seq, float eps) {
     if (!stream()) return QH_ESTATE;
     if (!qkv || !part || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
     if (max_seq <= 0 || max_seq > QM_MAX_SEQ) return QH_EINVAL;
-    const float scale = 0.08838834764831845f;   // 1 / sqrt(head_dim), qwen3.c:311
     hipLaunchKernelGGL(k_attn_part<QM_ATT_SPLITS>, dim3(NKV * QM_ATT_SPLITS), dim3(NTH), 0, stream(), qkv, part, kc, vc,
-                       qn, kn, rcos, rsin, pos_d, max_seq, (size_t)0, eps, scale);
+                       qn, kn, rcos, rsin, pos_d, max_seq, (size_t)0, eps, ATT_SCALE);
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 
+// Ranges per kv head: as few as keep each range of the longest context the
+// caches hold within one pass (64 positions), so that a pass is not mostly
+// padding; one range, which needs no merge, up to 128 positions once the
+// sequences make 64 blocks; at most QM_BATCH_SPLITS, whose blocks walk several
+// passes.  Measured on MI355X, graph-replayed, attention and merge against
+// eight ranges throughout: caches of 64 positions 5.8 / 9.8 / 23.7 -> 4.3 /
+// 4.9 / 7.9 us at 2 / 16 / 64 sequences, of 128 5.8 / 10.0 / 24.4 -> 5.7 / 6.9
+// / 12.5, of 224 5.9 / 11.1 / 26.2 -> 5.9 / 9.1 / 20.8; four ranges of 320
+// positions lose at 2 to 16 sequences (6.1 / 11.9 -> 7.7 / 12.5).
 extern "C" int qm_attention_decode_batch(const float *qkv, float *att, float *part, float *kc, float *vc,
                                          size_t kv_seq, const uint16_t *qn, const uint16_t *kn,
                                          const float *rcos, const float *rsin, const int *pos_d, int n_seq,
@@ -901,12 +933,11 @@ extern "C" int qm_attention_decode_batch(const float *qkv, float *att, float *pa
     if (!qkv || !att || !part || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
     if (n_seq <= 0 || n_seq > QM_MAX_CHUNK || max_seq <= 0 || max_seq > QM_MAX_SEQ) return QH_EINVAL;
     if (kv_seq < (size_t)NKV * HD * max_seq) return QH_EINVAL;     // sequences' caches must not overlap
-    const float scale = 0.08838834764831845f;   // 1 / sqrt(head_dim), qwen3.c:311
-    hipLaunchKernelGGL(k_attn_part<QM_BATCH_SPLITS>, dim3(NKV * QM_BATCH_SPLITS, n_seq), dim3(NTH), 0, stream(),
-                       qkv, part, kc, vc, qn, kn, rcos, rsin, pos_d, max_seq, kv_seq, eps, scale);
-    if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
-    hipLaunchKernelGGL(k_attn_merge<QM_BATCH_SPLITS>, dim3(NKV, n_seq), dim3(NTH), 0, stream(), att, part);
-    return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
+#define ATT_BATCH(S) launch_attn_decode<S>(qkv, att, part, kc, vc, kv_seq, qn, kn, rcos, rsin, pos_d, n_seq, max_seq, eps)
+    if (max_seq <= 64 || (max_seq <= 128 && NKV * n_seq >= 64)) return ATT_BATCH(1);
+    if (max_seq <= 256) return ATT_BATCH(4);
+    return ATT_BATCH(QM_BATCH_SPLITS);
+#undef ATT_BATCH
 }
 
 extern "C" int qm_argmax_rows(const float *logits, int n, int n_rows, int *tok, int *pos, const int *plen,

@@ -54,9 +54,9 @@ int qm_attention_decode_part(const float *qkv_d, float *part_d, float *kc_d, flo
 /* batched decode attention for n_seq sequences, one token each: row s of
  * qkv is sequence s's token at position pos[s]; its cache starts kv_seq
  * floats after sequence s-1's (same layout as above); each kv head's
- * positions are split into QM_BATCH_SPLITS ranges, whose partials (part:
- * QM_BATCH_PART_FLOATS per sequence) are merged into att[n_seq][2048]
- * (two launches) */
+ * positions are split into up to QM_BATCH_SPLITS ranges (fewer for a small
+ * max_seq), whose partials (part: QM_BATCH_PART_FLOATS per sequence) are
+ * merged into att[n_seq][2048] (two launches; one with a single range) */
 #ifndef QM_BATCH_SPLITS
 #define QM_BATCH_SPLITS 8
 #endif
