@@ -325,6 +325,16 @@ static inline bool m16_fits(int M, int K, int N) {
 // graph-replayed, 16 x 1024 x 8192 / 16384: 5.8 / 10.1 -> 4.5 / 7.7 us, and
 // 16 x 1024 x 4096: 3.8 -> 4.0 us the other way)
 static inline int m16_ct(int K, int N) { return K <= 2048 && (N + 15) / 16 > g_cus ? 2 : 1; }
+// places in k per block of the 16-row kernel (k_gemm_m16q): 4 or 8 columns per
+// block where those blocks make one round on the CUs, at K >= 2048 (measured on
+// MI355X, graph-replayed over weights that are not in any cache, M = 16: 3072 ->
+// 1024 7.6 -> 6.2 us, 2048 -> 1024 4.7 -> 4.2, 3072 -> 2048 8.0 -> 7.3, 2048 ->
+// 2048 5.8 -> 5.3; at K = 1024 nothing to gain, 3.1 -> 3.1 / 3.2; a second
+// round loses, 2048 -> 2048 on 4 columns 6.8, 3072 -> 3072 on 8 12.3 against 8.6)
+static inline int m16_nq(int K, int N) {
+    if (K < 2048) return 1;
+    return (N + 3) / 4 <= g_cus ? 4 : (N + 7) / 8 <= g_cus ? 2 : 1;
+}
 // the narrow kernel's limits: M <= 256, whole 128-deep slices, whole quads
 // of columns, byte offsets below 2 GiB; its geometry search also keeps the
 // tiles (row slab x 32 columns, a ticket each) within NARROW_CNT
@@ -1262,6 +1272,22 @@ static int launch_m16_t(float *c, const float *a, const uint16_t *b, const uint1
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
 }
+template <int NWV, int KT, int NQ>
+static int launch_m16q_t(float *c, const float *a, const uint16_t *b, int M, int N) {
+    constexpr int cols = 16 / NQ;
+    constexpr size_t lds = (size_t)16 * KT * 2 + (size_t)NWV * 16 * cols * sizeof(float);
+    static int attr_dev = -1;              // dynamic LDS above 64 KB must be opted into, per device
+    if (attr_dev != g_device) {
+        HCHECK(hipFuncSetAttribute((const void *)k_gemm_m16q<NWV, KT, NQ>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)lds),
+               QH_ELAUNCH);
+        attr_dev = g_device;
+    }
+    hipLaunchKernelGGL((k_gemm_m16q<NWV, KT, NQ>), dim3((unsigned)((N + cols - 1) / cols)), dim3(NWV * WAVE), lds,
+                       g_stream, c, a, b, M, N);
+    HCHECK(hipGetLastError(), QH_ELAUNCH);
+    return QH_OK;
+}
 // sizes within m16_fits (gated: K <= 2048), 16-byte aligned a, b, b2 (checked by the caller)
 template <bool GATED>
 static int launch_m16(float *c, const float *a, const uint16_t *b, const uint16_t *b2, int M, int K, int N) {
@@ -1272,6 +1298,13 @@ static int launch_m16(float *c, const float *a, const uint16_t *b, const uint16_
             default: return QH_EINVAL;
         }
     } else {
+        switch (K * 10 + m16_nq(K, N)) {
+            case 20482: return launch_m16q_t<8, 2048, 2>(c, a, b, M, N);
+            case 20484: return launch_m16q_t<8, 2048, 4>(c, a, b, M, N);
+            case 30722: return launch_m16q_t<8, 3072, 2>(c, a, b, M, N);
+            case 30724: return launch_m16q_t<8, 3072, 4>(c, a, b, M, N);
+            default: break;                        // 16 columns or more
+        }
         const int ct = m16_ct(K, N);
         switch (K * 10 + ct) {
             case 10241: return launch_m16_t<8, 1024, 1>(c, a, b, nullptr, M, N);

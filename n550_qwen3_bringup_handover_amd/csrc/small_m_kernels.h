@@ -989,4 +989,100 @@ __global__ __launch_bounds__(NWV * WAVE) void k_gemm_m16(float *__restrict__ c, 
     }
 }
 
+// ---------------------------------------------------------------------------
+// 16-row GEMM on narrow blocks: 16 / NQ columns of C per block
+// ---------------------------------------------------------------------------
+// The same as k_gemm_m16 for products with few columns (o and down of a small
+// decode batch), whose 16-column blocks leave most CUs idle.  A block owns COLS
+// = 16 / NQ columns; the 16 columns of the MFMA's B operand hold those COLS
+// weight rows at NQ places in k: lane (r, g) of step s holds chunk 4 NQ s + 4 q
+// + g (8 values of k) of weight row r % COLS, q = r / COLS.  A differs per
+// place, so step s is NQ MFMAs into NQ accumulators, of which accumulator q is
+// right in the columns of place q; the places are added across lanes at the
+// end.  The matrix cores do NQ times the useful work and stay idle most of the
+// time; a weight load instruction covers COLS rows x 64 NQ contiguous bytes and
+// lands in fragment order, so weights skip LDS.  Bound by the L2s' delivery of
+// A, which every block reads whole: 16 x 3072 fp32 to 256 blocks is 50 MB a
+// launch, about 3 of its 6.2 us (7.6 on 64 blocks of 16 columns, each reading
+// 98 KB of weights too; see m16_nq for the line).
+template <int NWV, int KT, int NQ>
+__global__ __launch_bounds__(NWV * WAVE) void k_gemm_m16q(float *__restrict__ c, const float *__restrict__ a,
+                                                          const uint16_t *__restrict__ b, int M, int N) {
+    constexpr int COLS = 16 / NQ, KW = KT / NWV, CHW = KW / 8, STEPS = CHW / (4 * NQ);
+    constexpr int PPR = KW / 4, APL = 16 * PPR / WAVE;   // 16-byte fp32 pieces of A per row / per lane
+    constexpr int SW = CHW >= 16 ? 15 : CHW - 1;
+    static_assert((NQ == 2 || NQ == 4) && KW * NWV == KT && STEPS * 4 * NQ == CHW && APL * WAVE == 16 * PPR, "k split");
+    extern __shared__ __align__(16) u32x4 m16_lds[];     // [NWV][16][CHW] A, [NWV][16][COLS] fp32 tiles
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    const int r16 = lane & 15, g = lane >> 4, q0 = r16 / COLS;
+    const int n0 = blockIdx.x * COLS;
+    u32x4 *const sa = m16_lds + w * 16 * CHW;
+    float *const red = reinterpret_cast<float *>(m16_lds + NWV * 16 * CHW);
+
+    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(b, (size_t)N * KT * 2);
+    u32x4 bw[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const int n = n0 + r16 % COLS;
+        const uint32_t off = n < N ? ((uint32_t)n * KT + w * KW + 8 * (4 * NQ * s + 4 * q0 + g)) * 2u : BUF_OOB;
+        bw[s] = __builtin_amdgcn_raw_buffer_load_b128(rb, off, 0, 0);
+    }
+    const __amdgpu_buffer_rsrc_t ra = buf_rsrc(a, (size_t)M * KT * 4);
+    u32x4 ap[APL];
+#pragma unroll
+    for (int j = 0; j < APL; j++) {
+        const int q = j * WAVE + lane, row = q / PPR, pc = q % PPR;
+        const uint32_t off = row < M ? ((uint32_t)row * KT + w * KW + 4 * pc) * 4u : BUF_OOB;
+        ap[j] = __builtin_amdgcn_raw_buffer_load_b128(ra, off, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < APL; j++) {
+        const int q = j * WAVE + lane, row = q / PPR, pc = q % PPR;
+        uint2 v;
+        v.x = pack_bf16x2(__uint_as_float(ap[j].x), __uint_as_float(ap[j].y));
+        v.y = pack_bf16x2(__uint_as_float(ap[j].z), __uint_as_float(ap[j].w));
+        *reinterpret_cast<uint2 *>(reinterpret_cast<unsigned char *>(sa + row * CHW + ((pc >> 1) ^ (row & SW))) +
+                                   8 * (pc & 1)) = v;
+    }
+    // only the wave itself reads its rows
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    f32x4 acc[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const int ch = 4 * NQ * s + 4 * q + g;
+            const bf16x8 af = __builtin_bit_cast(bf16x8, sa[r16 * CHW + (ch ^ (r16 & SW))]);
+            acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, __builtin_bit_cast(bf16x8, bw[s]), acc[q], 0, 0, 0);
+        }
+    // this lane's place, then the sum over places (columns r, r + COLS, ...)
+    f32x4 v = acc[0];
+#pragma unroll
+    for (int q = 1; q < NQ; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = q0 == q ? acc[q][r] : v[r];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        v[r] += dpp_partner<0x128>(v[r]);                  // row_ror:8
+        if constexpr (NQ == 4) v[r] += dpp_partner<0x124>(v[r]);   // row_ror:4
+    }
+    if (r16 < COLS) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[(w * 16 + 4 * g + r) * COLS + r16] = v[r];
+    }
+    __syncthreads();
+    if (threadIdx.x < 16 * COLS) {
+        const int m = threadIdx.x / COLS, n = n0 + threadIdx.x % COLS;
+        float sum = red[threadIdx.x];
+#pragma unroll
+        for (int u = 1; u < NWV; u++) sum += red[u * 16 * COLS + threadIdx.x];
+        if (m < M && n < N) c[(size_t)m * N + n] = sum;
+    }
+}
+
 #endif  // QH_SMALL_M_KERNELS_H
