@@ -802,7 +802,7 @@ static int launch_tile(float *c, const float *a, const uint16_t *b, const uint16
 // requires K % BK == 0 and 16-byte aligned a, b, b2 (checked by the caller)
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK = 32, int KG = 1>
 static int launch_pipe(float *c, const float *a, const uint16_t *b, const uint16_t *b2,
-                       int M, int K, int N) {
+                       int M, int K, int N, int slices = 1) {
     using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK, KG>;
     static int attr_dev = -1;              // dynamic LDS above 64 KB must be opted into, per device
     if (attr_dev != g_device) {
@@ -814,7 +814,7 @@ static int launch_pipe(float *c, const float *a, const uint16_t *b, const uint16
     TileMap map;
     const long tiles = make_map(map, M, N, K, BM, BN, R::BNO);
     if (tiles < 0) return QH_ETOOBIG;
-    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG>), dim3((unsigned)tiles, slices),
                        dim3(64 * WM * WN * KG), R::LDS, g_stream, c, a, b, b2, M, K, N, map);
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
@@ -1586,19 +1586,33 @@ extern "C" int qh_gemm_noalloc(float *c, const float *a, const uint16_t *b, int 
     return gemm_common(ws, true, c, a, b, nullptr, M, K, N, false);
 }
 
-// qh_gemm, except that when the skinny kernel splits K the slices' fp32 sums
-// are left in the split-K workspace ([ks][M][N], *part) for the caller to add
-// in slice order -- the sums k_stream_reduce would form -- instead of a second
-// launch.  Taken where the automatic plan is the skinny kernel, and for
-// M <= 128, K >= 2048, N <= 2048, where the kernel in 64-row slabs ties or
-// beats the 32x64 tiles once the reduction launch is gone (measured at
-// M = 96 / 128: down 13.2 / 13.2 -> ~9 us, o 9.6 / 9.8 -> ~6.5 us) -- but
-// not where the automatic plan is the narrow kernel, which writes C itself
-// (at M = 128 its o and down, with the plain residual + RMSNorm after them,
-// beat the split sums and the norm that adds them: 128-token prefill 1.68
-// -> 1.65 ms, 2,014-token prefill 40.3 -> 39.5 ms).
-// Otherwise C is written and *ks = 0.  The partials last until the next call
-// that uses the workspace.
+// K slices of the 32 x 64 ring tiles in qh_gemm_split (1: not taken): as many
+// whole slices of two or more 128-deep stages as keep the blocks within one
+// round.  The ring walks a block's stages one after the other, about half a us
+// each, so with few tiles a split shortens the chain; the residual + RMSNorm
+// that follows adds the slices.  Measured on MI355X, graph-replayed, weights
+// from HBM, GEMM and norm against the narrow kernel or one slice of the same
+// tiles: M = 128 o / down 10.6 / 12.3 -> 9.0 / 10.1 us, M = 160 11.7 / 16.0 ->
+// 10.0 / 10.9, M = 256 11.8 / 18.1 -> 10.4 / 13.6, M = 32 down 10.0 -> 8.6.  Up
+// to 64 rows at K = 2048 the narrow kernel stays (7.7 against 8.0 us), up to 16
+// the skinny kernel (16 x 3072 7.1 against 8.2).
+static int pipe_slices(int M, int K, int N) {
+    if (K % 128 || K < 2048 || N > 2048 || M <= 16 || (M <= 64 && K <= 2048)) return 1;
+    const long tiles = (long)((M + 31) / 32) * ((N + 63) / 64);
+    int best = 1;
+    for (int s = 2; s <= RMAX && s * tiles <= g_cus; s++)
+        if (K / 128 % s == 0 && K / 128 / s >= 2) best = s;
+    return best;
+}
+
+// qh_gemm, except that where a kernel splits K the slices' fp32 sums are left
+// in the split-K workspace ([ks][M][N], *part) for the caller to add in slice
+// order -- the sums k_stream_reduce would form -- instead of a second launch.
+// The 32 x 64 ring tiles where pipe_slices splits them; the skinny kernel where
+// it is the automatic plan or M <= 128, K >= 2048, N <= 2048 -- but not where
+// the automatic plan is the narrow kernel, which writes C itself.  Otherwise C
+// is written and *ks = 0.  The partials last until the next call that uses the
+// workspace.
 extern "C" int qh_gemm_split(float *c, const float *a, const uint16_t *b, int M, int K, int N,
                              const float **part, int *ks) {
     if (!part || !ks) return QH_EINVAL;
@@ -1606,21 +1620,26 @@ extern "C" int qh_gemm_split(float *c, const float *a, const uint16_t *b, int M,
     *ks = 0;
     if (!g_inited) return QH_ESTATE;
     const bool vec = M > 0 && K > 0 && N > 0 && a && b && c && (K % 8) == 0 && aligned16(a) && aligned16(b);
-    const int auto_plan = vec ? choose_plan(M, K, N, false, vec) : PLAN_SCALAR64;
-    const bool take = vec && !g_forced_plan && auto_plan != PLAN_NARROW &&
-                      (auto_plan == PLAN_SKINNY || (M <= 128 && K >= 2048 && N <= 2048));
     Ws ws = lib_ws();
-    if (take && M <= SKINNY_MMAX && K % 64 == 0 && (size_t)M * K * 4 < (1ull << 31) &&
-        (size_t)N * K * 2 < (1ull << 31)) {
-        const int s = skinny_slices(K, N, M);
+    if (vec && !g_forced_plan && (size_t)M * K * 4 < (1ull << 31) && (size_t)N * K * 2 < (1ull << 31)) {
+        const int auto_plan = choose_plan(M, K, N, false, vec);
+        int s = pipe_slices(M, K, N), plan = PLAN_P32x64k128s4;
+        if (s <= 1 && M <= SKINNY_MMAX && K % 64 == 0 && auto_plan != PLAN_NARROW &&
+            (auto_plan == PLAN_SKINNY || (M <= 128 && K >= 2048 && N <= 2048))) {
+            s = skinny_slices(K, N, M);
+            plan = PLAN_SKINNY;
+        }
         if (s > 1 && part_ensure(ws, (size_t)s * M * N * sizeof(float))) {
             int rc;
-            g_last_plan = PLAN_SKINNY;
-            switch (stream_mt(M)) {
-                case 1: rc = launch_skinny_t<1, false>(ws, c, a, b, nullptr, M, K, N, false); break;
-                case 2: rc = launch_skinny_t<2, false>(ws, c, a, b, nullptr, M, K, N, false); break;
-                default: rc = launch_skinny_t<4, false>(ws, c, a, b, nullptr, M, K, N, false); break;
-            }
+            g_last_plan = plan;
+            if (plan == PLAN_P32x64k128s4)
+                rc = launch_pipe<32, 64, 2, 2, 4, false, 128, 2>(use_part(ws), a, b, nullptr, M, K, N, s);
+            else
+                switch (stream_mt(M)) {
+                    case 1: rc = launch_skinny_t<1, false>(ws, c, a, b, nullptr, M, K, N, false); break;
+                    case 2: rc = launch_skinny_t<2, false>(ws, c, a, b, nullptr, M, K, N, false); break;
+                    default: rc = launch_skinny_t<4, false>(ws, c, a, b, nullptr, M, K, N, false); break;
+                }
             if (rc == QH_OK) {
                 *part = ws.part;
                 *ks = s;

@@ -330,6 +330,8 @@ template <int V> struct IC { static constexpr int value = V; };
 // 6.27; four groups from K = 2048: 512 x {2048, 3072} x 1024 9.5 / 12.7 ->
 // 9.1 / 12.2, but at K = 1024 they lose, 6.24 -> 6.35; 2 x 4 waves on the
 // plain tiles instead reached 6.75 / 10.6 / 14.5).
+// K split over blocks: blockIdx.y takes k range [y KB, (y + 1) KB), KB = K /
+// gridDim.y, and writes its sums as slice y of c ([gridDim.y][M][N]).
 template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_, int KG>
 __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__restrict__ c,
                                                           const float *__restrict__ a,
@@ -349,7 +351,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
     tile_of(blockIdx.x, map, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * R::BNO;
-    const int nk = K / R::BK;
+    const int nk = K / R::BK / (int)gridDim.y, kb0 = (int)blockIdx.y * nk * R::BK;
+    c += (size_t)blockIdx.y * M * N;
 
     const float *asrc[R::A_DMA];
     const uint16_t *bsrc[R::B_DMA];
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
         const int r = seg * (64 / R::CA) + lane / R::CA;
         const int cl = (lane % R::CA) ^ swz<R::CA>(r);
         const int gm = min(m0 + r, M - 1);
-        asrc[i] = a + (size_t)gm * K + cl * 4;
+        asrc[i] = a + (size_t)gm * K + kb0 + cl * 4;
     }
 #pragma unroll
     for (int i = 0; i < R::B_DMA; i++) {
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
             gn = n0 + r;
         }
         gn = min(gn, N - 1);
-        bsrc[i] = src + (size_t)gn * K + cl * 8;
+        bsrc[i] = src + (size_t)gn * K + kb0 + cl * 8;
     }
     // wave-uniform LDS byte offsets of this wave's copies within a slot
     const int a_dst = wave * R::A_DMA * 1024;
