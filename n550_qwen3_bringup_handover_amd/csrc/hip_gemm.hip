@@ -285,7 +285,11 @@ enum {
     // aligned (not gated)
     PLAN_R64x64 = 28,          // three register sets
     PLAN_R128x128 = 29,
-    PLAN_COUNT = 30
+    // bf16 A in the ring: tile, k per stage, eight waves in two k groups
+    PLAN_PB32x64k128 = 30,
+    PLAN_PB64x64k128 = 31,
+    PLAN_XB64x128 = 32,        // BK 64
+    PLAN_COUNT = 33
 };
 static const char *k_plan_names[PLAN_COUNT] = {
     "auto", "gemv", "mfma128x128", "mfma64x128", "mfma64x64", "mfma32x128", "mfma16x64", "mfma64x64-scalar",
@@ -293,12 +297,17 @@ static const char *k_plan_names[PLAN_COUNT] = {
     "xl128x128", "xl256x256", "xl64x128",
     "xb256x256k32", "xb128x128", "xb256x256s1",
     "stream", "stream-ks1", "stream-ks2", "stream-ks4", "stream-ks8", "skinny", "narrow", "wide",
-    "gemv16", "xl64x64s3", "m16", "rag64x64", "rag128x128"};
+    "gemv16", "xl64x64s3", "m16", "rag64x64", "rag128x128",
+    "pb32x64k128", "pb64x64k128", "xb64x128"};
 static inline bool is_pipe_plan(int p) { return p >= PLAN_P32x64k128s4 && p <= PLAN_P64x64k64s3; }
 static inline bool is_xl_plan(int p) {
-    return (p >= PLAN_X128x128 && p <= PLAN_XB256x256s1) || p == PLAN_X64x64s3;
+    return (p >= PLAN_X128x128 && p <= PLAN_XB256x256s1) || p == PLAN_X64x64s3 || p == PLAN_XB64x128;
 }
-static inline bool is_xb_plan(int p) { return p >= PLAN_XB256x256k32 && p <= PLAN_XB256x256s1; }
+static inline bool is_pb_plan(int p) { return p == PLAN_PB32x64k128 || p == PLAN_PB64x64k128; }
+// plans that read A as bf16
+static inline bool is_xb_plan(int p) {
+    return (p >= PLAN_XB256x256k32 && p <= PLAN_XB256x256s1) || p == PLAN_XB64x128 || is_pb_plan(p);
+}
 static inline bool is_stream_plan(int p) { return p >= PLAN_STREAM && p <= PLAN_STREAM_KS8; }
 static inline bool is_rag_plan(int p) { return p == PLAN_R64x64 || p == PLAN_R128x128; }
 // the ragged large tiles' limits: byte offsets below 2 GiB (their
@@ -375,18 +384,30 @@ static int stream_ks(int M, int K, int N, int cus) {
     return smallest;
 }
 static inline int xl_bk(int p) { return (p == PLAN_X256x256 || p == PLAN_XB256x256k32) ? 32 : 64; }
-static inline int pipe_bk(int p) { return p == PLAN_P32x64k128s4 ? 128 : 64; }
+static inline int pipe_bk(int p) {
+    return p == PLAN_P32x64k128s4 || is_pb_plan(p) ? 128 : 64;
+}
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-// bf16-A shapes: 256 x 256 tiles when they fill the chip, else the smaller
-// tiles (measured on MI355X for the Qwen3-0.6B projection shapes)
+// bf16-A shapes: the smallest tile that makes one round -- a CU takes in its
+// operands at 60 to 70 GB/s whatever the kernel, so what counts is the bytes of
+// a block and that every CU has one.  Measured on MI355X, graph-replayed over
+// weights that are not in any cache, against the 128 x 128 tiles: ring 32 x 64,
+// 128 / 512 x 3072 x 1024 23.8 / 23.6 -> 9.8 / 10.5 us and 128 x 1024 x 4096
+// 11.7 -> 6.4; ring 64 x 64, 256 x 1024 x 4096 13.0 -> 7.7, 1024 x 3072 x 1024
+// 23.6 -> 12.4, gate|up 128 rows 14.1 -> 8.8 (11.5 on 32 x 64, whose 32-row
+// blocks make more than a round); 64 x 128, 512 x 1024 x 4096 12.0 -> 9.9, 2048 x
+// 2048 x 1024 17.9 -> 15.4, gate|up 256 rows 14.0 -> 12.3.  Past a round of
+// those, 128 x 128, and 256 x 256 when they fill the chip.
 static int choose_bf16a_plan(int M, int K, int N, int gated) {
-    (void)K;
     const int bno = gated ? 2 : 1;
     auto blocks = [&](int bm, int bn) {
         return (long)((M + bm - 1) / bm) * (long)((N + bn / bno - 1) / (bn / bno));
     };
+    if (K % 128 == 0 && !gated && blocks(32, 64) <= g_cus) return PLAN_PB32x64k128;
+    if (K % 128 == 0 && blocks(64, 64) <= g_cus) return PLAN_PB64x64k128;
+    if (blocks(64, 128) <= g_cus) return PLAN_XB64x128;
     if (!gated && blocks(256, 256) >= 256) return PLAN_XB256x256k32;
     return PLAN_XB128x128;
 }
@@ -800,13 +821,13 @@ static int launch_tile(float *c, const float *a, const uint16_t *b, const uint16
 }
 
 // requires K % BK == 0 and 16-byte aligned a, b, b2 (checked by the caller)
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK = 32, int KG = 1>
-static int launch_pipe(float *c, const float *a, const uint16_t *b, const uint16_t *b2,
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK = 32, int KG = 1, bool ABF16 = false, bool SPLIT = false>
+static int launch_pipe(float *c, const void *a, const uint16_t *b, const uint16_t *b2,
                        int M, int K, int N, int slices = 1) {
-    using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK, KG>;
+    using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16>;
     static int attr_dev = -1;              // dynamic LDS above 64 KB must be opted into, per device
     if (attr_dev != g_device) {
-        HCHECK(hipFuncSetAttribute((const void *)k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG>,
+        HCHECK(hipFuncSetAttribute((const void *)k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, R::LDS),
                QH_ELAUNCH);
         attr_dev = g_device;
@@ -814,7 +835,7 @@ static int launch_pipe(float *c, const float *a, const uint16_t *b, const uint16
     TileMap map;
     const long tiles = make_map(map, M, N, K, BM, BN, R::BNO);
     if (tiles < 0) return QH_ETOOBIG;
-    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG>), dim3((unsigned)tiles, slices),
+    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT>), dim3((unsigned)tiles, slices),
                        dim3(64 * WM * WN * KG), R::LDS, g_stream, c, a, b, b2, M, K, N, map);
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
@@ -1379,6 +1400,9 @@ static int dispatch_bf16a(int p, float *c, const uint16_t *a, const uint16_t *b,
         case PLAN_XB256x256k32: return launch_xl<256, 256, 32, GATED, true>(c, a, b, b2, M, K, N);
         case PLAN_XB128x128:    return launch_xl<128, 128, 64, GATED, true>(c, a, b, b2, M, K, N);
         case PLAN_XB256x256s1:  return launch_xl<256, 256, 64, GATED, true, 1>(c, a, b, b2, M, K, N);
+        case PLAN_XB64x128:     return launch_xl<64, 128, 64, GATED, true>(c, a, b, b2, M, K, N);
+        case PLAN_PB32x64k128:  return launch_pipe<32, 64, 2, 2, 6, GATED, 128, 2, true>(c, a, b, b2, M, K, N);
+        case PLAN_PB64x64k128:  return launch_pipe<64, 64, 2, 2, 4, GATED, 128, 2, true>(c, a, b, b2, M, K, N);
         default: return QH_EINVAL;
     }
 }
@@ -1408,7 +1432,8 @@ static int dispatch(int plan, const Ws &ws, float *c, const float *a, const uint
                              : launch_pipe<32, 64, 2, 2, 4, GATED, 128, 2>(c, a, b, b2, M, K, N);
         case PLAN_P32x64k64s4:  return launch_pipe<32, 64, 2, 2, 4, GATED, 64>(c, a, b, b2, M, K, N);
         case PLAN_P64x64k64s3:  return launch_pipe<64, 64, 2, 2, 3, GATED, 64>(c, a, b, b2, M, K, N);
-        case PLAN_XB256x256k32: case PLAN_XB128x128: case PLAN_XB256x256s1: {
+        case PLAN_XB256x256k32: case PLAN_XB128x128: case PLAN_XB256x256s1: case PLAN_XB64x128:
+        case PLAN_PB32x64k128: case PLAN_PB64x64k128: {
             if ((size_t)M * K > ws.abf_elems) return QH_ETOOBIG;
             uint16_t *abf = use_abf(ws);
             const int rc = launch_cvt_bf16(abf, a, (size_t)M * K);
@@ -1451,7 +1476,7 @@ static int resolve_plan(Ws &ws, int M, int K, int N, bool gated, bool vec, bool 
     if (is_rag_plan(plan) && (gated || !rag_fits(M, K, N))) plan = vec ? PLAN_T64x64 : PLAN_SCALAR64;
     if (!vec && !is_rag_plan(plan)) plan = PLAN_SCALAR64;   // forced plans still need vector-safe inputs
     if (plan == PLAN_GEMV && (M > 4 || (size_t)M * K * 4 > 64 * 1024)) plan = PLAN_T64x64;
-    if (is_pipe_plan(plan) && (K % pipe_bk(plan)) != 0) plan = PLAN_T64x64;   // whole k stages
+    if ((is_pipe_plan(plan) || is_pb_plan(plan)) && (K % pipe_bk(plan)) != 0) plan = PLAN_T64x64;   // whole k stages
     if (plan == PLAN_X64x64s3 && gated) plan = PLAN_T64x64;   // one B block per wave tile
     if (is_xl_plan(plan) && ((K % xl_bk(plan)) != 0 ||           // xl copies whole k stages and
                              (size_t)M * K * 4 >= (1ull << 32) ||   // addresses with 32-bit offsets
@@ -1542,7 +1567,7 @@ static int gemm_bf16a_common(float *c, const uint16_t *a, const uint16_t *b, con
         return QH_EINVAL;
     if ((size_t)M * K * 2 >= (1ull << 32) || (size_t)N * K * 2 >= (1ull << 32)) return QH_ETOOBIG;
     int plan = g_forced_plan;
-    if (!is_xb_plan(plan)) plan = choose_bf16a_plan(M, K, N, gated);
+    if (!is_xb_plan(plan) || (is_pb_plan(plan) && K % pipe_bk(plan))) plan = choose_bf16a_plan(M, K, N, gated);
     g_last_plan = plan;
     return gated ? dispatch_bf16a<true>(plan, c, a, b, b2, M, K, N)
                  : dispatch_bf16a<false>(plan, c, a, b, nullptr, M, K, N);
@@ -1633,7 +1658,7 @@ extern "C" int qh_gemm_split(float *c, const float *a, const uint16_t *b, int M,
             int rc;
             g_last_plan = plan;
             if (plan == PLAN_P32x64k128s4)
-                rc = launch_pipe<32, 64, 2, 2, 4, false, 128, 2>(use_part(ws), a, b, nullptr, M, K, N, s);
+                rc = launch_pipe<32, 64, 2, 2, 4, false, 128, 2, false, true>(use_part(ws), a, b, nullptr, M, K, N, s);
             else
                 switch (stream_mt(M)) {
                     case 1: rc = launch_skinny_t<1, false>(ws, c, a, b, nullptr, M, K, N, false); break;

@@ -280,13 +280,14 @@ __device__ __forceinline__ int swz(int r) {
 // encoding: vmcnt bits [3:0] and [15:14]; expcnt and lgkmcnt left at max)
 #define QH_VMCNT(n) ((((n) & 15) | (((n) >> 4) << 14)) | (7 << 4) | (15 << 8))
 
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_ = 32, int KG = 1>
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_ = 32, int KG = 1, bool ABF16 = false>
 struct RingCfg {
     static constexpr int BK = BK_;                      // k per stage (32, 64, 128)
     static constexpr int KS = BK / 32;                  // MFMA k-steps per stage
     static constexpr int KSG = KS / KG;                 // ... per wave group
-    static constexpr int CA = BK / 4, CB = BK / 8;      // 16-byte chunks per A / B row
-    static constexpr int A_BYTES = BM * BK * 4, B_BYTES = BN * BK * 2;
+    static constexpr int AB = ABF16 ? 2 : 4;            // bytes of an A element
+    static constexpr int CA = BK * AB / 16, CB = BK / 8;   // 16-byte chunks per A / B row
+    static constexpr int A_BYTES = BM * BK * AB, B_BYTES = BN * BK * 2;
     static constexpr int STAGE = A_BYTES + B_BYTES;
     static constexpr int NW = WM * WN * KG;             // waves: KG groups of WM x WN
     static constexpr int A_DMA = A_BYTES / 1024 / NW;  // 1 KB copies per wave per step
@@ -330,15 +331,16 @@ template <int V> struct IC { static constexpr int value = V; };
 // 6.27; four groups from K = 2048: 512 x {2048, 3072} x 1024 9.5 / 12.7 ->
 // 9.1 / 12.2, but at K = 1024 they lose, 6.24 -> 6.35; 2 x 4 waves on the
 // plain tiles instead reached 6.75 / 10.6 / 14.5).
-// K split over blocks: blockIdx.y takes k range [y KB, (y + 1) KB), KB = K /
-// gridDim.y, and writes its sums as slice y of c ([gridDim.y][M][N]).
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_, int KG>
+// SPLIT: K split over blocks: blockIdx.y takes its K / gridDim.y of k and writes
+// its sums as slice blockIdx.y of c ([gridDim.y][M][N]).
+// ABF16: A is already bf16 (a points to its bits): half the bytes, no conversion.
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_, int KG, bool ABF16 = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__restrict__ c,
-                                                          const float *__restrict__ a,
+                                                          const void *__restrict__ a,
                                                           const uint16_t *__restrict__ b,
                                                           const uint16_t *__restrict__ b2,
                                                           int M, int K, int N, TileMap map) {
-    using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK_, KG>;
+    using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK_, KG, ABF16>;
     static_assert(STAGES >= 3, "one stage being read, one in use, one or more in flight");
     extern __shared__ __align__(16) unsigned char smem[];
 
@@ -351,10 +353,11 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
     tile_of(blockIdx.x, map, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * R::BNO;
-    const int nk = K / R::BK / (int)gridDim.y, kb0 = (int)blockIdx.y * nk * R::BK;
-    c += (size_t)blockIdx.y * M * N;
+    const int nk = SPLIT ? K / R::BK / (int)gridDim.y : K / R::BK;
+    const int kb0 = SPLIT ? (int)blockIdx.y * nk * R::BK : 0;
+    if constexpr (SPLIT) c += (size_t)blockIdx.y * M * N;
 
-    const float *asrc[R::A_DMA];
+    const unsigned char *asrc[R::A_DMA];
     const uint16_t *bsrc[R::B_DMA];
 #pragma unroll
     for (int i = 0; i < R::A_DMA; i++) {
@@ -362,7 +365,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
         const int r = seg * (64 / R::CA) + lane / R::CA;
         const int cl = (lane % R::CA) ^ swz<R::CA>(r);
         const int gm = min(m0 + r, M - 1);
-        asrc[i] = a + (size_t)gm * K + kb0 + cl * 4;
+        asrc[i] = (const unsigned char *)a + ((size_t)gm * K + kb0) * R::AB + cl * 16;
     }
 #pragma unroll
     for (int i = 0; i < R::B_DMA; i++) {
@@ -391,7 +394,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
 #pragma unroll
         for (int i = 0; i < R::A_DMA; i++)
             __builtin_amdgcn_global_load_lds(
-                (const void *)(asrc[i] + k0),
+                (const void *)(asrc[i] + k0 * R::AB),
                 (__attribute__((address_space(3))) void *)(slot + a_dst + i * 1024), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < R::B_DMA; i++)
@@ -416,7 +419,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
         brow_sw[j] = swz<R::CB>(row);
     }
 
-    u32x4 fa[2][R::KSG][R::TM][2], fb[2][R::KSG][R::TN];
+    u32x4 fa[2][R::KSG][R::TM][ABF16 ? 1 : 2], fb[2][R::KSG][R::TN];
     // `SET` selects the register set at compile time (IC<0> / IC<1>)
     auto read_frags = [&](int step, auto SET) {
         constexpr int set = decltype(SET)::value;
@@ -427,8 +430,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
 #pragma unroll
             for (int i = 0; i < R::TM; i++) {
                 const u32x4 *rowp = reinterpret_cast<const u32x4 *>(slot + arow_off[i]);
-                fa[set][tt][i][0] = rowp[(8 * t + 2 * lgrp) ^ arow_sw[i]];
-                fa[set][tt][i][1] = rowp[(8 * t + 2 * lgrp + 1) ^ arow_sw[i]];
+                if constexpr (ABF16) {
+                    fa[set][tt][i][0] = rowp[(4 * t + lgrp) ^ arow_sw[i]];
+                } else {
+                    fa[set][tt][i][0] = rowp[(8 * t + 2 * lgrp) ^ arow_sw[i]];
+                    fa[set][tt][i][1] = rowp[(8 * t + 2 * lgrp + 1) ^ arow_sw[i]];
+                }
             }
 #pragma unroll
             for (int j = 0; j < R::TN; j++) {
@@ -451,8 +458,12 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
             bf16x8 af[R::TM];
 #pragma unroll
             for (int i = 0; i < R::TM; i++) {
+                if constexpr (ABF16) {
+                    af[i] = __builtin_bit_cast(bf16x8, fa[set][t][i][0]);
+                    continue;
+                }
                 const f32x4 x0 = __builtin_bit_cast(f32x4, fa[set][t][i][0]);
-                const f32x4 x1 = __builtin_bit_cast(f32x4, fa[set][t][i][1]);
+                const f32x4 x1 = __builtin_bit_cast(f32x4, fa[set][t][i][ABF16 ? 0 : 1]);
                 u32x4 w;
                 w.x = pack_bf16x2(x0.x, x0.y);
                 w.y = pack_bf16x2(x0.z, x0.w);
