@@ -543,6 +543,15 @@ static int choose_plan(int M, int K, int N, int gated, bool vec) {
         if (!gated && M >= 256 && blocks(64, 128) >= 192 && blocks(64, 128) <= g_cus) return PLAN_X64x128;
         if (!gated && M >= 512 && blocks(128, 128) >= 192 && blocks(128, 128) <= g_cus) return PLAN_X128x128;
         if (!gated && M > 128 && blocks(64, 64) >= 192 && blocks(64, 64) <= g_cus) return PLAN_X64x64s3;
+        // between 512 and 1024 rows the ring tiles below make more than a round,
+        // so the same two tiles with fewer blocks too (weights from HBM, against
+        // the register-staged 64 x 64 tiles: 520 x {1024, 2048, 3072} x 1024
+        // 15.8 / 31.6 / 45.7 -> 8.6 / 17.6 / 23.8 us, 600 x 2048 x 2048 32.2 ->
+        // 20.1 on 64 x 128)
+        if (!gated && M > 512 && M < 1024) {
+            if (blocks(64, 64) <= g_cus) return PLAN_X64x64s3;
+            if (blocks(64, 128) <= g_cus) return PLAN_X64x128;
+        }
         // gated between 128 and 512 rows where 128 x 128 tiles would leave
         // half the chip idle, and between 512 and 1024: 64 x 128 tiles (256 x
         // 1024 x 3072: 15.3 -> 10.4 us against the 64 x 64 tiles; 768 / 1024
