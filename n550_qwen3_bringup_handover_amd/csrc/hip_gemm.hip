@@ -830,13 +830,14 @@ static int launch_tile(float *c, const float *a, const uint16_t *b, const uint16
 }
 
 // requires K % BK == 0 and 16-byte aligned a, b, b2 (checked by the caller)
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK = 32, int KG = 1, bool ABF16 = false, bool SPLIT = false>
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK = 32, int KG = 1, bool ABF16 = false, bool SPLIT = false,
+          bool CBF16 = false>
 static int launch_pipe(float *c, const void *a, const uint16_t *b, const uint16_t *b2,
                        int M, int K, int N, int slices = 1) {
     using R = RingCfg<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16>;
     static int attr_dev = -1;              // dynamic LDS above 64 KB must be opted into, per device
     if (attr_dev != g_device) {
-        HCHECK(hipFuncSetAttribute((const void *)k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT>,
+        HCHECK(hipFuncSetAttribute((const void *)k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT, CBF16>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, R::LDS),
                QH_ELAUNCH);
         attr_dev = g_device;
@@ -844,7 +845,7 @@ static int launch_pipe(float *c, const void *a, const uint16_t *b, const uint16_
     TileMap map;
     const long tiles = make_map(map, M, N, K, BM, BN, R::BNO);
     if (tiles < 0) return QH_ETOOBIG;
-    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT>), dim3((unsigned)tiles, slices),
+    hipLaunchKernelGGL((k_gemm_pipe<BM, BN, WM, WN, STAGES, GATED, BK, KG, ABF16, SPLIT, CBF16>), dim3((unsigned)tiles, slices),
                        dim3(64 * WM * WN * KG), R::LDS, g_stream, c, a, b, b2, M, K, N, map);
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
@@ -966,7 +967,7 @@ static Ws lib_ws(void) { return Ws{g_abf, g_abf_elems, g_part, g_part_bytes, tru
 // -> 17.6; 64 x 128 tiles 2048 x 1024 x 1024 12.8 -> 11.3).  With more
 // tiles than CUs, two blocks of four waves per CU stay faster (gated M =
 // 1024 26.4 against 33.3 us).
-template <int BM, int BN, int BK, bool GATED, bool ABF16 = false, int SETS = 2>
+template <int BM, int BN, int BK, bool GATED, bool ABF16 = false, int SETS = 2, bool CBF16 = false>
 static int launch_xl(float *c, const void *a, const uint16_t *b, const uint16_t *b2,
                      int M, int K, int N) {
     using X = XlCfg<BM, BN, BK, GATED, ABF16, SETS>;
@@ -975,7 +976,7 @@ static int launch_xl(float *c, const void *a, const uint16_t *b, const uint16_t 
     if (tiles < 0) return QH_ETOOBIG;
     if constexpr (GATED && BM == 128 && BN == 128) {
         if (tiles <= g_cus) {
-            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 4, 1, 0>), dim3((unsigned)tiles, 1),
+            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 4, 1, 0, CBF16>), dim3((unsigned)tiles, 1),
                                dim3(XlCfg<BM, BN, BK, GATED, ABF16, SETS, 4>::NT), 0, g_stream, c, a, b, b2, M, K, N,
                                map);
             HCHECK(hipGetLastError(), QH_ELAUNCH);
@@ -984,14 +985,14 @@ static int launch_xl(float *c, const void *a, const uint16_t *b, const uint16_t 
     }
     if constexpr (BK == 64 && BM * BN <= 128 * 128 && (!GATED || BM * BN < 128 * 128)) {
         if (tiles <= g_cus) {
-            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 2, 0>), dim3((unsigned)tiles, 1),
+            hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 2, 0, CBF16>), dim3((unsigned)tiles, 1),
                                dim3(XlCfg<BM, BN, BK, GATED, ABF16, SETS, 2, 2>::NT), 0, g_stream, c, a, b, b2, M, K, N,
                                map);
             HCHECK(hipGetLastError(), QH_ELAUNCH);
             return QH_OK;
         }
     }
-    hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 1, 0>), dim3((unsigned)tiles, 1), dim3(X::NT), 0,
+    hipLaunchKernelGGL((k_gemm_xl<BM, BN, BK, GATED, ABF16, SETS, 2, 1, 0, CBF16>), dim3((unsigned)tiles, 1), dim3(X::NT), 0,
                        g_stream, c, a, b, b2, M, K, N, map);
     HCHECK(hipGetLastError(), QH_ELAUNCH);
     return QH_OK;
@@ -1417,6 +1418,18 @@ static int dispatch_bf16a(int p, float *c, const uint16_t *a, const uint16_t *b,
 }
 
 
+// gate|up with bf16 A and bf16 C, on the tiles choose_bf16a_plan picks for it
+static int dispatch_bf16ac(int p, uint16_t *h, const uint16_t *a, const uint16_t *b, const uint16_t *b2, int M, int K,
+                           int N) {
+    float *c = reinterpret_cast<float *>(h);
+    switch (p) {
+        case PLAN_PB64x64k128: return launch_pipe<64, 64, 2, 2, 4, true, 128, 2, true, false, true>(c, a, b, b2, M, K, N);
+        case PLAN_XB64x128:    return launch_xl<64, 128, 64, true, true, 2, true>(c, a, b, b2, M, K, N);
+        case PLAN_XB128x128:   return launch_xl<128, 128, 64, true, true, 2, true>(c, a, b, b2, M, K, N);
+        default: return QH_EINVAL;
+    }
+}
+
 template <bool GATED>
 static int dispatch(int plan, const Ws &ws, float *c, const float *a, const uint16_t *b, const uint16_t *b2,
                     int M, int K, int N) {
@@ -1541,6 +1554,25 @@ static int resolve_plan(Ws &ws, int M, int K, int N, bool gated, bool vec, bool 
     return plan;
 }
 
+// K slices of the 32 x 64 ring tiles in qh_gemm_split (1: not taken): as many
+// whole slices of two or more 128-deep stages as keep the blocks within one
+// round.  The ring walks a block's stages one after the other, about half a us
+// each, so with few tiles a split shortens the chain; the residual + RMSNorm
+// that follows adds the slices.  Measured on MI355X, graph-replayed, weights
+// from HBM, GEMM and norm against the narrow kernel or one slice of the same
+// tiles: M = 128 o / down 10.6 / 12.3 -> 9.0 / 10.1 us, M = 160 11.7 / 16.0 ->
+// 10.0 / 10.9, M = 256 11.8 / 18.1 -> 10.4 / 13.6, M = 32 down 10.0 -> 8.6.  Up
+// to 64 rows at K = 2048 the narrow kernel stays (7.7 against 8.0 us), up to 16
+// the skinny kernel (16 x 3072 7.1 against 8.2).
+static int pipe_slices(int M, int K, int N) {
+    if (K % 128 || K < 2048 || N > 2048 || M <= 16 || (M <= 64 && K <= 2048)) return 1;
+    const long tiles = (long)((M + 31) / 32) * ((N + 63) / 64);
+    int best = 1;
+    for (int s = 2; s <= RMAX && s * tiles <= g_cus; s++)
+        if (K / 128 % s == 0 && K / 128 / s >= 2) best = s;
+    return best;
+}
+
 static int gemm_common(Ws ws, bool strict, float *c, const float *a, const uint16_t *b, const uint16_t *b2,
                        int M, int K, int N, bool gated) {
     if (!g_inited) return QH_ESTATE;
@@ -1591,6 +1623,40 @@ extern "C" int qh_gemm_gate_up_silu_bf16a(float *h, const uint16_t *x, const uin
     return gemm_bf16a_common(h, x, wg, wu, M, K, N, true);
 }
 
+extern "C" int qh_gemm_gate_up_silu_bf16ac(uint16_t *h, const uint16_t *x, const uint16_t *wg, const uint16_t *wu,
+                                           int M, int K, int N) {
+    if (!g_inited) return QH_ESTATE;
+    if (!h || !x || !wg || !wu || M <= 0 || N <= 0 || K <= 0 || K % 64 || !aligned16(x) || !aligned16(wg) || !aligned16(wu))
+        return QH_EINVAL;
+    if ((size_t)M * K * 2 >= (1ull << 32) || (size_t)N * K * 2 >= (1ull << 32)) return QH_ETOOBIG;
+    g_last_plan = choose_bf16a_plan(M, K, N, 1);
+    return dispatch_bf16ac(g_last_plan, h, x, wg, wu, M, K, N);
+}
+
+// qh_gemm_bf16a that may leave K slices unadded, as qh_gemm_split
+extern "C" int qh_gemm_split_bf16a(float *c, const uint16_t *a, const uint16_t *b, int M, int K, int N,
+                                   const float **part, int *ks) {
+    if (!part || !ks) return QH_EINVAL;
+    *part = nullptr;
+    *ks = 0;
+    if (!g_inited) return QH_ESTATE;
+    if (M > 0 && N > 0 && K > 0 && c && a && b && K % 128 == 0 && aligned16(a) && aligned16(b) &&
+        (size_t)N * K * 2 < (1ull << 31)) {
+        Ws ws = lib_ws();
+        const int s = pipe_slices(M, K, N);
+        if (s > 1 && part_ensure(ws, (size_t)s * M * N * sizeof(float))) {
+            g_last_plan = PLAN_PB32x64k128;
+            const int rc = launch_pipe<32, 64, 2, 2, 6, false, 128, 2, true, true>(use_part(ws), a, b, nullptr, M, K, N, s);
+            if (rc == QH_OK) {
+                *part = ws.part;
+                *ks = s;
+            }
+            return rc;
+        }
+    }
+    return gemm_bf16a_common(c, a, b, nullptr, M, K, N, false);
+}
+
 extern "C" int qh_gemm(float *c, const float *a, const uint16_t *b, int M, int K, int N) {
     return gemm_common(lib_ws(), false, c, a, b, nullptr, M, K, N, false);
 }
@@ -1618,25 +1684,6 @@ extern "C" int qh_gemm_noalloc(float *c, const float *a, const uint16_t *b, int 
     const Ws ws{(uint16_t *)s, QH_SCRATCH_WS_BYTES / sizeof(uint16_t), (float *)s, QH_SCRATCH_WS_BYTES, false,
                 (unsigned *)((unsigned char *)s + QH_SCRATCH_WS_BYTES)};
     return gemm_common(ws, true, c, a, b, nullptr, M, K, N, false);
-}
-
-// K slices of the 32 x 64 ring tiles in qh_gemm_split (1: not taken): as many
-// whole slices of two or more 128-deep stages as keep the blocks within one
-// round.  The ring walks a block's stages one after the other, about half a us
-// each, so with few tiles a split shortens the chain; the residual + RMSNorm
-// that follows adds the slices.  Measured on MI355X, graph-replayed, weights
-// from HBM, GEMM and norm against the narrow kernel or one slice of the same
-// tiles: M = 128 o / down 10.6 / 12.3 -> 9.0 / 10.1 us, M = 160 11.7 / 16.0 ->
-// 10.0 / 10.9, M = 256 11.8 / 18.1 -> 10.4 / 13.6, M = 32 down 10.0 -> 8.6.  Up
-// to 64 rows at K = 2048 the narrow kernel stays (7.7 against 8.0 us), up to 16
-// the skinny kernel (16 x 3072 7.1 against 8.2).
-static int pipe_slices(int M, int K, int N) {
-    if (K % 128 || K < 2048 || N > 2048 || M <= 16 || (M <= 64 && K <= 2048)) return 1;
-    const long tiles = (long)((M + 31) / 32) * ((N + 63) / 64);
-    int best = 1;
-    for (int s = 2; s <= RMAX && s * tiles <= g_cus; s++)
-        if (K / 128 % s == 0 && K / 128 / s >= 2) best = s;
-    return best;
 }
 
 // qh_gemm, except that where a kernel splits K the slices' fp32 sums are left

@@ -99,12 +99,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, size_t
 //       xb[row] = rmsnorm(x[row]) * nw           (ops_scalar.c:11-16)
 // grid = nt blocks of 256 threads; K % 4 == 0, K <= 4096, ks <= KS_MAX.
 // ---------------------------------------------------------------------------
+// BF: xb is bf16 (RNE), the rounding the product that reads it applies anyway.
 #define KS_MAX 16
+// four floats to bf16, RNE
+__device__ __forceinline__ uint2 pack4(f32x4 v) {
+    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(uint2, __builtin_convertvector(v, bf4));
+}
+template <bool BF>
 __global__ __launch_bounds__(NTH) void k_rows_norm(float *__restrict__ x, const float *__restrict__ r,
                                                    const uint16_t *__restrict__ emb,
                                                    const int *__restrict__ tok, int emb_rows,
                                                    const uint16_t *__restrict__ nw,
-                                                   float *__restrict__ xb, int K, float eps,
+                                                   void *__restrict__ xb, int K, float eps,
                                                    const float *__restrict__ part, int ks, size_t pstride) {
     const int row = blockIdx.x, tid = threadIdx.x;
     const int n4 = K >> 2;
@@ -162,7 +169,8 @@ __global__ __launch_bounds__(NTH) void k_rows_norm(float *__restrict__ x, const 
             o.y = (v[j].y * scale) * bf16f(w[1]);
             o.z = (v[j].z * scale) * bf16f(w[2]);
             o.w = (v[j].w * scale) * bf16f(w[3]);
-            reinterpret_cast<f32x4 *>(xb + (size_t)row * K)[c] = o;
+            if constexpr (BF) reinterpret_cast<uint2 *>((uint16_t *)xb + (size_t)row * K)[c] = pack4(o);
+            else reinterpret_cast<f32x4 *>((float *)xb + (size_t)row * K)[c] = o;
         }
     }
 }
@@ -245,9 +253,10 @@ __global__ __launch_bounds__(NTH) void k_rope_cache(const float *__restrict__ qk
 
 __device__ __forceinline__ bool not_finite(float x) { return (__float_as_uint(x) & 0x7F800000u) == 0x7F800000u; }
 
-template <int MT, int NW>
+// BF: out is bf16 (RNE), the rounding the o projection applies anyway.
+template <int MT, int NW, bool BF>
 __global__ __launch_bounds__(WAVE * NW, 2) void k_attn_chunk(const float *__restrict__ qkv,
-                                                             float *__restrict__ out, float *__restrict__ part,
+                                                             void *__restrict__ out, float *__restrict__ part,
                                                              const float *__restrict__ kc,
                                                              const float *__restrict__ vc,
                                                              const uint16_t *__restrict__ qn,
@@ -452,7 +461,8 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_attn_chunk(const float *__rest
         }
         const size_t orow = (size_t)(i0 + (row >> 1)) * (NKV * GRP) + g * GRP + (row & 1);   // [token][head]
         if (gridDim.y == 1) {
-            reinterpret_cast<f32x4 *>(out + orow * HD)[d4] = acc / L;
+            if constexpr (BF) reinterpret_cast<uint2 *>((uint16_t *)out + orow * HD)[d4] = pack4(acc / L);
+            else reinterpret_cast<f32x4 *>((float *)out + orow * HD)[d4] = acc / L;
         } else {
             float *pp = part + ((size_t)blockIdx.y * nt * (NKV * GRP) + orow) * ATT_LD;
             reinterpret_cast<f32x4 *>(pp)[d4] = acc;
@@ -464,7 +474,8 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_attn_chunk(const float *__rest
 // the key splits' partials part[ks][token][head][ATT_LD] (sums, max at HD,
 // weight at HD + 1) merged into out[token][head][HD].  One block of 128
 // threads per 4 (token, head) rows, a thread per 4 dims.
-__global__ __launch_bounds__(128) void k_attn_chunk_merge(float *__restrict__ out, const float *__restrict__ part,
+template <bool BF>
+__global__ __launch_bounds__(128) void k_attn_chunk_merge(void *__restrict__ out, const float *__restrict__ part,
                                                           int rows, int ks) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 5), d4 = threadIdx.x & 31;
     if (row >= rows) return;
@@ -489,7 +500,8 @@ __global__ __launch_bounds__(128) void k_attn_chunk_merge(float *__restrict__ ou
             L = fmaf(wt, l[s], L);
             acc += wt * v[s];
         }
-    reinterpret_cast<f32x4 *>(out + (size_t)row * HD)[d4] = acc / L;
+    if constexpr (BF) reinterpret_cast<uint2 *>((uint16_t *)out + (size_t)row * HD)[d4] = pack4(acc / L);
+    else reinterpret_cast<f32x4 *>((float *)out + (size_t)row * HD)[d4] = acc / L;
 }
 
 // ---------------------------------------------------------------------------
@@ -838,23 +850,33 @@ __global__ void k_zero_i32(int *p, int n) {
 // ---------------------------------------------------------------------------
 static inline hipStream_t stream() { return (hipStream_t)qh_stream(); }
 
-extern "C" int qm_rows_norm(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
-                            const uint16_t *nw, float *xb, int nt, int K, float eps) {
-    return qm_rows_norm_split(x, r, emb, tok, emb_rows, nw, xb, nt, K, eps, nullptr, 0);
-}
-
-extern "C" int qm_rows_norm_split(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
-                                  const uint16_t *nw, float *xb, int nt, int K, float eps, const float *part,
-                                  int ks) {
+template <bool BF>
+static int rows_norm(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows, const uint16_t *nw,
+                     void *xb, int nt, int K, float eps, const float *part, int ks) {
     if (!stream()) return QH_ESTATE;
     if (!x || !nw || !xb || nt <= 0 || K <= 0 || K % 4 || K > 4 * 4 * NTH) return QH_EINVAL;
     if (emb && (!tok || emb_rows <= 0)) return QH_EINVAL;
     if (ks < 0 || ks > KS_MAX || (ks > 0 && (!part || emb || r))) return QH_EINVAL;
     const size_t pstride = (size_t)nt * K;                  // one slice: [nt][K]
     if (ks > 0 && pstride * ks * 4 >= ((size_t)1 << 31)) return QH_EINVAL;
-    hipLaunchKernelGGL(k_rows_norm, dim3(nt), dim3(NTH), 0, stream(), x, emb ? nullptr : r, emb, tok,
+    hipLaunchKernelGGL(k_rows_norm<BF>, dim3(nt), dim3(NTH), 0, stream(), x, emb ? nullptr : r, emb, tok,
                        emb_rows, nw, xb, K, eps, part, ks, pstride);
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
+}
+
+extern "C" int qm_rows_norm_split(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
+                                  const uint16_t *nw, float *xb, int nt, int K, float eps, const float *part,
+                                  int ks) {
+    return rows_norm<false>(x, r, emb, tok, emb_rows, nw, xb, nt, K, eps, part, ks);
+}
+extern "C" int qm_rows_norm_bf16(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
+                                 const uint16_t *nw, uint16_t *xb, int nt, int K, float eps, const float *part,
+                                 int ks) {
+    return rows_norm<true>(x, r, emb, tok, emb_rows, nw, xb, nt, K, eps, part, ks);
+}
+extern "C" int qm_rows_norm(float *x, const float *r, const uint16_t *emb, const int *tok, int emb_rows,
+                            const uint16_t *nw, float *xb, int nt, int K, float eps) {
+    return rows_norm<false>(x, r, emb, tok, emb_rows, nw, xb, nt, K, eps, nullptr, 0);
 }
 
 // The chunk attention's launch: 16-token blocks (each K and V load feeding two
@@ -862,9 +884,10 @@ extern "C" int qm_rows_norm_split(float *x, const float *r, const uint16_t *emb,
 // waves below; the context split over blocks while the grid leaves CUs idle
 // and every wave would walk at least ATT_SPLIT_TILES key tiles.
 #define ATT_SPLIT_TILES 4
-extern "C" int qm_attention(const float *qkv, float *out, float *part, float *kc, float *vc, const uint16_t *qn,
-                            const uint16_t *kn, const float *rcos, const float *rsin, const int *pos_d,
-                            int nt, int max_seq, int ctx_bound, float eps) {
+template <bool BF>
+static int attention(const float *qkv, void *out, float *part, float *kc, float *vc, const uint16_t *qn,
+                     const uint16_t *kn, const float *rcos, const float *rsin, const int *pos_d, int nt, int max_seq,
+                     int ctx_bound, float eps) {
     if (!stream()) return QH_ESTATE;
     if (!qkv || !out || !part || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
     if (nt <= 0 || max_seq <= 0 || nt > max_seq || max_seq > QM_MAX_SEQ) return QH_EINVAL;
@@ -874,20 +897,31 @@ extern "C" int qm_attention(const float *qkv, float *out, float *part, float *kc
     if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
     const int tiles = (ctx_bound + 15) / 16;
     if ((nt + 15) / 16 * NKV >= 256) {
-        hipLaunchKernelGGL((k_attn_chunk<2, 4>), dim3((nt + 15) / 16 * NKV), dim3(4 * WAVE), 0, stream(), qkv, out,
+        hipLaunchKernelGGL((k_attn_chunk<2, 4, BF>), dim3((nt + 15) / 16 * NKV), dim3(4 * WAVE), 0, stream(), qkv, out,
                            part, kc, vc, qn, rcos, rsin, pos_d, nt, max_seq, eps);
         return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
     }
     const int blocks = (nt + 7) / 8 * NKV;
     int ks = 1;
     while (ks < ATT_KS && nt <= QM_ATT_KS_ROWS && 2 * ks * blocks <= 256 && tiles >= 8 * ks * ATT_SPLIT_TILES) ks *= 2;
-    hipLaunchKernelGGL((k_attn_chunk<1, 8>), dim3(blocks, ks), dim3(8 * WAVE), 0, stream(), qkv, out, part, kc, vc,
+    hipLaunchKernelGGL((k_attn_chunk<1, 8, BF>), dim3(blocks, ks), dim3(8 * WAVE), 0, stream(), qkv, out, part, kc, vc,
                        qn, rcos, rsin, pos_d, nt, max_seq, eps);
     if (hipGetLastError() != hipSuccess) return QH_ELAUNCH;
     if (ks > 1)
-        hipLaunchKernelGGL(k_attn_chunk_merge, dim3(nt * (NKV * GRP) / 4), dim3(128), 0, stream(), out, part,
+        hipLaunchKernelGGL(k_attn_chunk_merge<BF>, dim3(nt * (NKV * GRP) / 4), dim3(128), 0, stream(), out, part,
                            nt * NKV * GRP, ks);
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
+}
+
+extern "C" int qm_attention(const float *qkv, float *out, float *part, float *kc, float *vc, const uint16_t *qn,
+                            const uint16_t *kn, const float *rcos, const float *rsin, const int *pos_d,
+                            int nt, int max_seq, int ctx_bound, float eps) {
+    return attention<false>(qkv, out, part, kc, vc, qn, kn, rcos, rsin, pos_d, nt, max_seq, ctx_bound, eps);
+}
+extern "C" int qm_attention_bf16(const float *qkv, uint16_t *out, float *part, float *kc, float *vc, const uint16_t *qn,
+                                 const uint16_t *kn, const float *rcos, const float *rsin, const int *pos_d,
+                                 int nt, int max_seq, int ctx_bound, float eps) {
+    return attention<true>(qkv, out, part, kc, vc, qn, kn, rcos, rsin, pos_d, nt, max_seq, ctx_bound, eps);
 }
 
 // n_seq sequences' decode attention in S ranges per kv head, merged into att

@@ -91,6 +91,12 @@ int qh_gemm_bf16a(float *c_d, const uint16_t *a_d, const uint16_t *b_d,
                   int M, int K, int N);
 int qh_gemm_gate_up_silu_bf16a(float *h_d, const uint16_t *x_d, const uint16_t *wg_d,
                                const uint16_t *wu_d, int M, int K, int N);
+/* the gated product with bf16 h too (RNE), for a caller that rounds it anyway */
+int qh_gemm_gate_up_silu_bf16ac(uint16_t *h_d, const uint16_t *x_d, const uint16_t *wg_d,
+                                const uint16_t *wu_d, int M, int K, int N);
+/* qh_gemm_bf16a that may leave K slices unadded, as qh_gemm_split */
+int qh_gemm_split_bf16a(float *c_d, const uint16_t *a_d, const uint16_t *b_d, int M, int K, int N,
+                        const float **part_d, int *ks);
 /* tile-major [N/tn][K/tk][tn][tk] -> row-major [N][K] */
 int qh_tile_to_row(uint16_t *dst_d, const uint16_t *src_d, int N, int K,
                    int tile_n, int tile_k);

@@ -26,6 +26,11 @@ int qm_rows_norm_split(float *x_d, const float *r_d, const uint16_t *emb_d, cons
                        const uint16_t *nw_d, float *xb_d, int nt, int K, float eps, const float *part_d,
                        int ks);
 
+/* the same with bf16 xb (RNE), for products that round it anyway */
+int qm_rows_norm_bf16(float *x_d, const float *r_d, const uint16_t *emb_d, const int *tok_d, int emb_rows,
+                      const uint16_t *nw_d, uint16_t *xb_d, int nt, int K, float eps, const float *part_d,
+                      int ks);
+
 /* QK-norm + RoPE + KV-cache write, then causal GQA attention, for nt tokens
  * at positions *pos_d .. *pos_d + nt - 1 of one layer (two launches, three
  * where a short chunk's context is split over blocks).  ctx_bound (host-known,
@@ -39,6 +44,10 @@ int qm_rows_norm_split(float *x_d, const float *r_d, const uint16_t *emb_d, cons
 int qm_attention(const float *qkv_d, float *out_d, float *part_d, float *kc_d, float *vc_d,
                  const uint16_t *qn_d, const uint16_t *kn_d, const float *rcos_d, const float *rsin_d,
                  const int *pos_d, int nt, int max_seq, int ctx_bound, float eps);
+/* the same with bf16 out (RNE) */
+int qm_attention_bf16(const float *qkv_d, uint16_t *out_d, float *part_d, float *kc_d, float *vc_d,
+                      const uint16_t *qn_d, const uint16_t *kn_d, const float *rcos_d, const float *rsin_d,
+                      const int *pos_d, int nt, int max_seq, int ctx_bound, float eps);
 
 /* decode attention split into QM_ATT_SPLITS position ranges per kv head:
  * writes softmax partials (m, l, o[128] per head and range, QM_ATT_PART

@@ -311,6 +311,13 @@ struct RingCfg {
 // ---------------------------------------------------------------------------
 template <int V> struct IC { static constexpr int value = V; };
 
+// element i of a gated product's C, fp32 or bf16
+template <bool CBF16>
+__device__ __forceinline__ void store_gated(float *c, size_t i, float v) {
+    if constexpr (CBF16) reinterpret_cast<uint16_t *>(c)[i] = __builtin_bit_cast(uint16_t, (__bf16)v);
+    else __builtin_nontemporal_store(v, &c[i]);
+}
+
 // A and B stream straight into an LDS ring of STAGES slots with
 // global_load_lds (16-byte copies, explicit vmcnt waits, one barrier per
 // stage), and the phases of consecutive stages overlap inside each wave: while the MFMAs of stage `it` run on
@@ -334,7 +341,9 @@ template <int V> struct IC { static constexpr int value = V; };
 // SPLIT: K split over blocks: blockIdx.y takes its K / gridDim.y of k and writes
 // its sums as slice blockIdx.y of c ([gridDim.y][M][N]).
 // ABF16: A is already bf16 (a points to its bits): half the bytes, no conversion.
-template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_, int KG, bool ABF16 = false, bool SPLIT = false>
+// CBF16 (gated): C is stored as bf16 (RNE), for a product that rounds it anyway.
+template <int BM, int BN, int WM, int WN, int STAGES, bool GATED, int BK_, int KG, bool ABF16 = false, bool SPLIT = false,
+          bool CBF16 = false>
 __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__restrict__ c,
                                                           const void *__restrict__ a,
                                                           const uint16_t *__restrict__ b,
@@ -589,8 +598,8 @@ __global__ __launch_bounds__(64 * WM * WN * KG, 1) void k_gemm_pipe(float *__res
 #pragma unroll
                     for (int r = 0; r < 4; r++)
                         if (rbase + r < M)
-                            __builtin_nontemporal_store(silu_mul(acc[i][j][r], acc[i][j + TNO][r]),
-                                                        &c[(size_t)(rbase + r) * N + col]);
+                            store_gated<CBF16>(c, (size_t)(rbase + r) * N + col,
+                                               silu_mul(acc[i][j][r], acc[i][j + TNO][r]));
                 }
             }
         }
@@ -743,7 +752,8 @@ typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 // element, out of range past K.  Only the last stage differs, and it is loaded
 // in the prologue or the tail, so the steady loop is the aligned kernel's.
 // RAG 1 and 2 need A and B below 2 GiB each (the out-of-range marker).
-template <int BM, int BN, int BK, bool GATED, bool ABF16, int SETS, int WMW, int KG, int RAG>
+// CBF16 (gated): C is stored as bf16.
+template <int BM, int BN, int BK, bool GATED, bool ABF16, int SETS, int WMW, int KG, int RAG, bool CBF16 = false>
 __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) * KG == 8 ? 1 : (BM * BN <= 128 * 128 ? 2 : 1)) void k_gemm_xl(float *__restrict__ c,
                                                         const void *__restrict__ a,
                                                         const uint16_t *__restrict__ b,
@@ -1094,8 +1104,7 @@ __global__ __launch_bounds__(64 * WMW * xl_wn(BM, BN) * KG, WMW * xl_wn(BM, BN) 
                     for (int v = 0; v < 16; v++) {
                         const int row = rbase + 8 * (v >> 2) + (v & 3);
                         if (row < M)
-                            __builtin_nontemporal_store(silu_mul(acc[i][j][v], acc[i][j + TNO][v]),
-                                                        &c[(size_t)row * N + col]);
+                            store_gated<CBF16>(c, (size_t)row * N + col, silu_mul(acc[i][j][v], acc[i][j + TNO][v]));
                     }
                 }
             }
