@@ -108,7 +108,8 @@ int qwen3_hip_model_set_graph(qwen3_hip_model *model, int on);
  * the environment makes 1 the default); both give the same bits (no
  * counterpart in the reference, which has no launches).  On MI355X the
  * persistent launch measured 3% slower (1,720-1,750 against 1,780-1,805
- * tok/s for 128 greedy steps after a 128-token prompt).  Turning it on where
+ * tok/s for 128 greedy steps after a 128-token prompt).  Steps whose context
+ * exceeds 1,024 positions are per-layer launches in either mode.  Turning it on where
  * the device cannot keep the launch's 256 workgroups resident returns
  * QWEN3_HIP_ENODEV.  qwen3_hip_model_persistent returns the mode. */
 int qwen3_hip_model_set_persistent(qwen3_hip_model *model, int on);

@@ -34,7 +34,7 @@ static hipEvent_t g_ev[64];
 static int g_ev_made[64];
 static int g_forced_plan = 0;
 static int g_last_plan = 0;        // the plan the last GEMM call launched (PLAN_AUTO: none yet)
-#define QH_MAX_GRAPHS 16
+#define QH_MAX_GRAPHS 32        // a model holds two, a batch one
 static hipGraphExec_t g_graph_exec[QH_MAX_GRAPHS];
 static void *g_graph_ws[QH_MAX_GRAPHS][2];   // library workspaces each graph uses (abf, part)
 // Workspaces replaced while a graph exists: a captured graph keeps the device

@@ -950,6 +950,21 @@ extern "C" int qm_attention_decode_part(const float *qkv, float *part, float *kc
     return hipGetLastError() == hipSuccess ? QH_OK : QH_ELAUNCH;
 }
 
+// One sequence's decode attention behind more than QM_LONG_CTX positions: 64
+// blocks (eight ranges) read 60 GB/s each and walk ctx / 512 passes, so twice
+// the ranges, merged by a launch of their own (in the o GEMV every block reads
+// all partials again).  Measured on MI355X, graph-replayed, attention, merge and
+// o GEMV: context 1,816 13.5 -> 11.5 us, 4,000 21.3 -> 16.2, 8,000 36.2 -> 23.8;
+// 1,000 9.8 -> 9.4, 500 7.6 -> 9.1 the other way.
+extern "C" int qm_attention_decode_long(const float *qkv, float *att, float *part, float *kc, float *vc,
+                                        const uint16_t *qn, const uint16_t *kn, const float *rcos, const float *rsin,
+                                        const int *pos_d, int max_seq, float eps) {
+    if (!stream()) return QH_ESTATE;
+    if (!qkv || !att || !part || !kc || !vc || !qn || !kn || !rcos || !rsin || !pos_d) return QH_EINVAL;
+    if (max_seq <= 0 || max_seq > QM_MAX_SEQ) return QH_EINVAL;
+    return launch_attn_decode<QM_ATT_LONG_SPLITS>(qkv, att, part, kc, vc, 0, qn, kn, rcos, rsin, pos_d, 1, max_seq, eps);
+}
+
 // Ranges per kv head: as few as keep each range of the longest context the
 // caches hold within one pass (64 positions), so that a pass is not mostly
 // padding; one range, which needs no merge, up to 128 positions once the

@@ -50,14 +50,14 @@ struct qwen3_hip_model {
     float *kc, *vc;                    /* [NL][KVH][..] see hip_model.hip */
     float *rcos, *rsin;                /* [max_seq][64] */
     float *x, *x0, *x1, *xb, *qkv, *att, *ob, *hb, *dn, *logits;
-    float *apart;                      /* decode attention partials [QM_ATT_PART_FLOATS] */
+    float *apart;                      /* decode attention partials [QM_ATT_LONG_PART_FLOATS] */
     float *cpart;                      /* chunk attention partials [QM_ATT_CHUNK_PART_FLOATS] */
     int *tok_in;                       /* [prefill_rows(max_seq)] */
     int *state;                        /* [0] token, [1] position, [2] step */
     int *out_tok;                      /* [max_seq + 1] */
     int use_graph;
     int use_persist;                   /* decode layers as one persistent launch */
-    int graph_id;                      /* -1 until captured */
+    int graph_id[2];                   /* the decode step (1: long context), -1 until captured */
     qwen3_hip_dump_fn dump;            /* chunk-path intermediate dumps (NULL = off) */
     void *dump_ctx;
     float *dump_host;                  /* staging for dumps */
@@ -141,7 +141,8 @@ void qwen3_hip_model_close(qwen3_hip_model *m) {
     if (!m) return;
     (void)qh_sync();
     detach_batches(m);
-    if (m->graph_id >= 0) (void)qh_graph_destroy(m->graph_id);
+    for (int g = 0; g < 2; g++)
+        if (m->graph_id[g] >= 0) (void)qh_graph_destroy(m->graph_id[g]);
     void *bufs[] = {m->wbuf, m->kc, m->vc, m->rcos, m->rsin, m->x, m->x0, m->x1, m->xb, m->qkv,
                     m->att, m->ob, m->hb, m->dn, m->logits, m->apart, m->cpart, m->tok_in, m->state, m->out_tok};
     for (size_t i = 0; i < sizeof bufs / sizeof bufs[0]; i++) (void)qh_free(bufs[i]);
@@ -164,7 +165,7 @@ int qwen3_hip_model_open(qwen3_hip_model **out, const void *blob, size_t size, i
     if (!m) return QWEN3_HIP_ENOMEM;
     m->max_seq = max_seq;
     m->use_graph = 1;
-    m->graph_id = -1;
+    m->graph_id[0] = m->graph_id[1] = -1;
     {
         /* the persistent decode launch, opt-in: measured slower than the
          * per-layer launches (1,720-1,750 against 1,780-1,805 tok/s).  Its
@@ -196,7 +197,7 @@ int qwen3_hip_model_open(qwen3_hip_model **out, const void *blob, size_t size, i
     DEV(m->hb, B * QW3M_INTER * 4);
     DEV(m->dn, B * H * 4);
     DEV(m->logits, (size_t)V * 4);
-    DEV(m->apart, (size_t)QM_ATT_PART_FLOATS * 4);
+    DEV(m->apart, (size_t)QM_ATT_LONG_PART_FLOATS * 4);
     DEV(m->cpart, QM_ATT_CHUNK_PART_FLOATS * 4);
     DEV(m->tok_in, B * sizeof(int));
     DEV(m->state, 4 * sizeof(int));
@@ -311,11 +312,11 @@ int qwen3_hip_model_set_persistent(qwen3_hip_model *m, int on) {
         if (rc) return rc;
         if (!qm_persist_supported()) return QWEN3_HIP_ENODEV;
     }
-    if ((on ? 1 : 0) != m->use_persist && m->graph_id >= 0) {   /* the captured step is the other kind */
+    if ((on ? 1 : 0) != m->use_persist && m->graph_id[0] >= 0) {   /* the captured step is the other kind */
         int rc = qh_sync();
-        if (!rc) rc = qh_graph_destroy(m->graph_id);
+        if (!rc) rc = qh_graph_destroy(m->graph_id[0]);
         if (rc) return rc;
-        m->graph_id = -1;
+        m->graph_id[0] = -1;
     }
     m->use_persist = on ? 1 : 0;
     return QWEN3_HIP_OK;
@@ -450,9 +451,12 @@ static int run_chunk(qwen3_hip_model *m, const kv_t *kv, int nt, int pos0, int w
 }
 
 /* the logits of token state[0] at position state[1], its K and V appended to
- * the cache; the layers as one launch when persist */
-static int decode_logits(qwen3_hip_model *m, int persist) {
+ * the cache; the layers as one launch when persist, except behind a long
+ * context (more than QM_LONG_CTX positions, the new one included), whose
+ * attention is split finer than that launch does */
+static int decode_logits(qwen3_hip_model *m, int persist, int lng) {
     int rc = QWEN3_HIP_OK;
+    persist = persist && !lng;
     const float eps = QW3M_RMS_EPS;
     if (persist) {
         /* the 28 layers in one launch: x0 and dn as the per-layer launches leave them */
@@ -470,11 +474,17 @@ static int decode_logits(qwen3_hip_model *m, int persist) {
         qh_gemv_pro_t pro = {m->x0, NULL, NULL, 0, m->dn, L->in_norm, m->x1, eps};
         if (l == 0) { pro.x = NULL; pro.r = NULL; pro.emb = m->embed; pro.tok = m->state; pro.emb_rows = V; }
         rc = qh_gemv_pro(m->qkv, &pro, L->wqkv, NULL, H, QKV_N, 0);
-        /* attention as split-softmax partials, merged in the o GEMV's prologue */
-        if (!rc) rc = qm_attention_decode_part(m->qkv, m->apart, m->kc + l * kv_layer_floats(m),
-                                               m->vc + l * kv_layer_floats(m), L->qn, L->kn, m->rcos,
-                                               m->rsin, m->state + 1, m->max_seq, eps);
-        if (!rc) rc = qh_gemv_merge(m->ob, m->apart, L->wo, QW3M_Q_DIM, H);
+        float *kc = m->kc + l * kv_layer_floats(m), *vc = m->vc + l * kv_layer_floats(m);
+        if (lng) {
+            if (!rc) rc = qm_attention_decode_long(m->qkv, m->att, m->apart, kc, vc, L->qn, L->kn, m->rcos, m->rsin,
+                                                   m->state + 1, m->max_seq, eps);
+            if (!rc) rc = qh_gemm(m->ob, m->att, L->wo, 1, QW3M_Q_DIM, H);
+        } else {
+            /* attention as split-softmax partials, merged in the o GEMV's prologue */
+            if (!rc) rc = qm_attention_decode_part(m->qkv, m->apart, kc, vc, L->qn, L->kn, m->rcos, m->rsin,
+                                                   m->state + 1, m->max_seq, eps);
+            if (!rc) rc = qh_gemv_merge(m->ob, m->apart, L->wo, QW3M_Q_DIM, H);
+        }
         const qh_gemv_pro_t pro2 = {m->x1, NULL, NULL, 0, m->ob, L->post_norm, m->x0, eps};
         if (!rc) rc = qh_gemv_pro(m->hb, &pro2, L->wg, L->wu, H, QW3M_INTER, 1);
         if (!rc) rc = qh_gemm(m->dn, m->hb, L->wd, 1, QW3M_INTER, H);
@@ -486,8 +496,8 @@ static int decode_logits(qwen3_hip_model *m, int persist) {
 
 /* one greedy decode step on the device: token state[0] at position
  * state[1]; appends the next token to out_tok[state[2]] */
-static int decode_step(qwen3_hip_model *m) {
-    int rc = decode_logits(m, m->use_persist);
+static int decode_step(qwen3_hip_model *m, int lng) {
+    int rc = decode_logits(m, m->use_persist, lng);
     if (!rc) rc = qh_argmax_step(m->state, m->out_tok, m->state + 2, m->max_seq + 1, m->state + 1, 1,
                                  m->logits, V);
     return rc;
@@ -536,7 +546,7 @@ int qwen3_hip_model_forward(qwen3_hip_model *m, const int *tokens, int n_token, 
            launches per layer on the GEMV kernels instead of a chunk's eight
            (measured on MI355X behind 700 positions: 1,255 -> 655 us a call) */
         rc = qm_set_tokens(m->state, tokens, 1, m->state + 1, pos0);
-        if (!rc) rc = decode_logits(m, 0);
+        if (!rc) rc = decode_logits(m, 0, pos0 + 1 > QM_LONG_CTX);
     } else if (!rc) {
         const kv_t kv = model_kv(m);
         rc = load_chunk(m, tokens, n_token, pos0);
@@ -581,20 +591,27 @@ int qwen3_hip_model_generate(qwen3_hip_model *m, const int *prompt, int n_prompt
     const double t1 = now_ms();
     if (rc) return rc;
 
-    if (n_decode > 0 && m->use_graph && m->graph_id < 0) {
-        rc = qh_capture_begin();
-        if (!rc) {
-            int rc2 = decode_step(m);
+    for (int s = 0; s < n_decode && !rc; s++) {
+        const int lng = n_prompt + s + 1 > QM_LONG_CTX;
+        if (m->use_graph && m->graph_id[lng] < 0) {
+            rc = qh_capture_begin();
+            if (rc) break;
+            const int rc2 = decode_step(m, lng);
             int gid = -1;
             rc = qh_capture_end(&gid);
             if (!rc) rc = rc2;
-            if (!rc) m->graph_id = gid;
-            else if (gid >= 0) (void)qh_graph_destroy(gid);
+            if (rc) {
+                if (gid >= 0) (void)qh_graph_destroy(gid);
+                break;
+            }
+            m->graph_id[lng] = gid;
         }
-        if (rc) return rc;
+        rc = m->use_graph ? qh_graph_launch(m->graph_id[lng]) : decode_step(m, lng);
     }
-    for (int s = 0; s < n_decode && !rc; s++)
-        rc = m->use_graph ? qh_graph_launch(m->graph_id) : decode_step(m);
+    if (rc) {
+        (void)qh_sync();               /* steps already launched */
+        return rc;
+    }
     if (!rc) rc = qh_sync();
     const double t2 = now_ms();
     if (rc) return rc;

@@ -60,6 +60,16 @@ int qm_attention_decode_part(const float *qkv_d, float *part_d, float *kc_d, flo
                              const uint16_t *qn_d, const uint16_t *kn_d, const float *rcos_d,
                              const float *rsin_d, const int *pos_d, int max_seq, float eps);
 
+/* the same for a long context (more than QM_LONG_CTX positions):
+ * QM_ATT_LONG_SPLITS ranges, merged into att[2048] by a second launch (part:
+ * QM_ATT_LONG_PART_FLOATS) */
+#define QM_LONG_CTX 1024
+#define QM_ATT_LONG_SPLITS 16
+#define QM_ATT_LONG_PART_FLOATS (8 * QM_ATT_LONG_SPLITS * 2 * QM_ATT_PART)
+int qm_attention_decode_long(const float *qkv_d, float *att_d, float *part_d, float *kc_d, float *vc_d,
+                             const uint16_t *qn_d, const uint16_t *kn_d, const float *rcos_d,
+                             const float *rsin_d, const int *pos_d, int max_seq, float eps);
+
 /* batched decode attention for n_seq sequences, one token each: row s of
  * qkv is sequence s's token at position pos[s]; its cache starts kv_seq
  * floats after sequence s-1's (same layout as above); each kv head's
