@@ -235,7 +235,8 @@ __global__ __launch_bounds__(NTH) void k_rope_cache(const float *__restrict__ qk
 // during its S product, the next tile's K loads during its P V product.
 // Positions past a row's own context score -inf and weigh 0; a V entry that
 // is not finite must not reach the rows that do not see it (0 * inf), so
-// tiles on the diagonal look for one and then keep such rows' sums apart.
+// tiles on the diagonal look for one and then leave it out of such rows' sums,
+// row by row.
 // grid = (ceil(nt / (8 MT)) * NKV, KS): block b takes kv head b % NKV, so each
 // XCD (b mod 8) serves one head's K and V from its own L2, and the token
 // tiles with the longest contexts first.
@@ -400,28 +401,26 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_attn_chunk(const float *__rest
                     for (int mt = 0; mt < MT; mt++)
                         o[mt][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][dt >> 2][dt & 3], pr[mt][r], o[mt][dt], 0, 0, 0);
         } else {
-            // the first position of the tile with such an entry: rows that
-            // see it take every V as it is, the others none that is not finite
-            int tmin = 0x7FFFFFFF;
-#pragma unroll
-            for (int r = 3; r >= 0; r--) {
-                bool b = false;
-#pragma unroll
-                for (int e = 0; e < 8; e++) b |= not_finite(vv[r][e >> 2][e & 3]);
-                if (b) tmin = 16 * kt + 4 * h + r;
-            }
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) tmin = min(tmin, __shfl_xor(tmin, d));
+            // every row takes the entries up to its own position as they are and
+            // the later ones that are not finite as 0: one product per token of
+            // the row tile, of which its rows keep the result
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int dt = 0; dt < 8; dt++) {
-                    const float v = vv[r][dt >> 2][dt & 3], vz = not_finite(v) ? 0.0f : v;
+                    const float v = vv[r][dt >> 2][dt & 3];
+                    const bool bad = not_finite(v);
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++) {
-                        const f32x4 a = __builtin_amdgcn_mfma_f32_16x16x4f32(v, pr[mt][r], o[mt][dt], 0, 0, 0);
-                        const f32x4 z = __builtin_amdgcn_mfma_f32_16x16x4f32(vz, pr[mt][r], o[mt][dt], 0, 0, 0);
-                        o[mt][dt] = tmin <= pos0 + i0 + 8 * mt + (c >> 1) ? a : z;
+                        const int p0 = pos0 + i0 + 8 * mt;
+                        f32x4 keep = o[mt][dt];
+#pragma unroll 1
+                        for (int u = 0; u < 8; u++) {
+                            const float vu = bad && 16 * kt + 4 * h + r > p0 + u ? 0.0f : v;
+                            const f32x4 w = __builtin_amdgcn_mfma_f32_16x16x4f32(vu, pr[mt][r], o[mt][dt], 0, 0, 0);
+                            keep = (c >> 1) == u ? w : keep;
+                        }
+                        o[mt][dt] = keep;
                     }
                 }
         }

@@ -127,3 +127,26 @@ def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(nt, pos0):
     assert np.array_equal(got[:j], clean[:j])
     assert not np.isfinite(got[j:, 4:6, 5]).any()
     assert np.array_equal(np.delete(got[j], [4, 5], 0), np.delete(clean[j], [4, 5], 0))
+
+
+@pytest.mark.parametrize("nt,pos0,cached", [(24, 0, ()), (24, 605, (600,)), (600, 0, ()), (600, 5, (3,))])
+def test_several_values_that_are_not_finite_in_one_tile(nt, pos0, cached):
+    """Two or three positions of one 16-position tile on the diagonal hold an
+    entry that is not finite, each in a dim of its own (one of them may lie in
+    the cache): every row gets those at and before its own position, and its
+    other outputs are those without such entries, bit for bit."""
+    x = Case(nt, pos0, pos0 + nt)
+    clean = x.run()[0]
+    bad = [(p, 7) for p in cached]
+    for t in cached:
+        x.v[2, t, 7] = np.nan
+    first = 0 if pos0 else 13
+    for n, j in enumerate((first, first + 1, first + 2)):
+        x.qkv[j, 3072 + 2 * HD + 9 + n] = (np.inf, -np.inf, np.nan)[n]
+        bad.append((pos0 + j, 9 + n))
+    got = x.run()[0]
+    rows = pos0 + np.arange(nt)
+    for p, d in bad:
+        assert np.array_equal(np.isfinite(got[:, 4:6, d]).all(1), rows < p), (p, d)
+        got[rows >= p, 4:6, d] = clean[rows >= p, 4:6, d]
+    assert np.array_equal(got, clean)
