@@ -494,8 +494,8 @@ __global__ __launch_bounds__(128) void k_attn_chunk_merge(void *__restrict__ out
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < ATT_KS; s++)
-        if (m[s] != -INFINITY) {
-            const float wt = expf(m[s] - M);
+        if (s < ks) {                                    // a NaN weight stays one under wt = 0
+            const float wt = m[s] == -INFINITY ? 0.0f : expf(m[s] - M);
             L = fmaf(wt, l[s], L);
             acc += wt * v[s];
         }

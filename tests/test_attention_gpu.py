@@ -150,3 +150,17 @@ def test_several_values_that_are_not_finite_in_one_tile(nt, pos0, cached):
         assert np.array_equal(np.isfinite(got[:, 4:6, d]).all(1), rows < p), (p, d)
         got[rows >= p, 4:6, d] = clean[rows >= p, 4:6, d]
     assert np.array_equal(got, clean)
+
+
+@pytest.mark.parametrize("nt,pos0,splits", [(24, 600, 2), (1, 2047, 8), (24, 16, 1)])
+def test_scores_that_are_nan_stay_in_the_sum(nt, pos0, splits):
+    """NaN keys at every position of the second key split (of eight waves with
+    one split): a range whose maximum is -inf because all its scores are NaN is
+    not an empty one."""
+    x = Case(nt, pos0, pos0 + nt)
+    clean = x.run()[0]
+    tile = np.arange(pos0) // 16 % (8 * splits)
+    x.k[2, (tile >= 8) & (tile < 16) if splits > 1 else tile == 0] = np.nan
+    got = x.run()[0]
+    assert np.isnan(got[:, 4:6]).all()
+    assert np.array_equal(np.delete(got, [4, 5], 1), np.delete(clean, [4, 5], 1))
