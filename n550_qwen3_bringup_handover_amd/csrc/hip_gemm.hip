@@ -1782,6 +1782,8 @@ extern "C" int qh_capture_end(int *graph_id) {
     return QH_OK;
 }
 
+extern "C" int qh_capturing(void) { return g_capturing; }
+
 extern "C" int qh_graph_launch(int id) {
     if (!g_inited) return QH_ESTATE;
     if (id < 0 || id >= QH_MAX_GRAPHS || !g_graph_exec[id]) return QH_EINVAL;

@@ -155,6 +155,7 @@ int qh_read(const void *src_d, size_t bytes);
  * into a graph that qh_graph_launch replays on the shim stream */
 int qh_capture_begin(void);
 int qh_capture_end(int *graph_id);
+int qh_capturing(void);            /* 1 between the two */
 int qh_graph_launch(int graph_id);
 int qh_graph_destroy(int graph_id);
 

@@ -511,8 +511,10 @@ static int check_tokens(const int *t, int n) {
 
 /* tokens -> tok_in and pos0 -> state[1].  Up to QM_MAX_CHUNK tokens travel as
  * kernel arguments: no copy and no wait (a copy from the caller's pageable
- * memory has to be waited for) */
+ * memory has to be waited for).  Refused while the caller records a graph: its
+ * replays would feed these tokens again */
 static int load_chunk(qwen3_hip_model *m, const int *tokens, int nt, int pos0) {
+    if (qh_capturing()) return QWEN3_HIP_ERUNTIME;
     if (nt <= QM_MAX_CHUNK) return qm_set_tokens(m->tok_in, tokens, nt, m->state + 1, pos0);
     int rc = qh_h2d(m->tok_in, tokens, (size_t)nt * sizeof(int));
     if (!rc) rc = qm_set_i32(m->state + 1, pos0);
@@ -545,7 +547,7 @@ int qwen3_hip_model_forward(qwen3_hip_model *m, const int *tokens, int n_token, 
         /* one token is a decode step whose next token the caller picks: five
            launches per layer on the GEMV kernels instead of a chunk's eight
            (measured on MI355X behind 700 positions: 1,255 -> 655 us a call) */
-        rc = qm_set_tokens(m->state, tokens, 1, m->state + 1, pos0);
+        rc = qh_capturing() ? QWEN3_HIP_ERUNTIME : qm_set_tokens(m->state, tokens, 1, m->state + 1, pos0);
         if (!rc) rc = decode_logits(m, 0, pos0 + 1 > QM_LONG_CTX);
     } else if (!rc) {
         const kv_t kv = model_kv(m);

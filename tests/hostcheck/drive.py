@@ -10,6 +10,8 @@ the stand-in's report and exit with its violation count.
                        workspace growth, 48 rotating weight copies)
     drive.py selftest  a deliberate misuse (a buffer freed while a live graph
                        uses it, then the graph launched): must be reported
+    drive.py capture   forward, generate and batch prefill while the caller
+                       records a graph: refused, nothing recorded
     drive.py model     the device-resident forward and batched decode on a
                        small cache: prefill, greedy generate (graph replay),
                        batch prefill/decode (graph replay), re-prefill
@@ -96,6 +98,42 @@ def run_model():
             say(f"batch of {n_seq}")
 
 
+def run_capture():
+    """Calls that take tokens from the host are not for a graph: each is
+    refused between capture_begin and capture_end, before it launches
+    anything, and the graph that is recorded around them holds only the
+    caller's own product."""
+    import bench
+    import numpy as np
+    from n550_qwen3_bringup_handover_amd import model as M
+    g = bench.Gpu()
+    a, c, w = g.alloc(4 * 1024), g.alloc(4 * 1024), g.alloc(2 * 1024 * 1024)
+    with M.Model(M.qw3m_random(0x03550040, M.LAYOUT_ROW, threads=8), max_seq=256) as m, M.Batch(m, 2, 200) as b:
+        toks = np.arange(150, dtype=np.int32)
+        calls = [lambda n=n: m.forward(toks[:n], 3) for n in (1, 2, 64, 65, 128)]
+        calls += [lambda n=n: m.generate(toks[:n], 2) for n in (1, 128, 150)]
+        calls += [lambda n=n: b.prefill(1, toks[:n]) for n in (1, 150)]
+        for i, call in enumerate(calls):
+            g.rt.check(g.L.qwen3_hip_capture_begin(), "capture_begin")
+            g.gemm(c, a, w, 1, 1024, 1024)
+            n = STUB.hipstub_recorded()
+            try:
+                call()
+                sys.exit(f"call {i} was taken while a graph is recorded")
+            except runtime.Qwen3HipError as e:
+                say(f"call {i}: {e}")
+            if STUB.hipstub_recorded() != n:
+                sys.exit(f"call {i} left {STUB.hipstub_recorded() - n} launches in the graph")
+            gid = ctypes.c_int(-1)
+            g.rt.check(g.L.qwen3_hip_capture_end(ctypes.byref(gid)), "capture_end")
+            g.rt.check(g.L.qwen3_hip_graph_launch(gid.value), "graph_launch")
+            g.rt.check(g.L.qwen3_hip_graph_destroy(gid.value), "graph_destroy")
+        m.forward(toks[:1], 3)
+        m.generate(toks, 2)
+    for p in (a, c, w):
+        g.rt.check(g.L.qwen3_hip_free(ctypes.c_void_p(p)), "free")
+
+
 def run_selftest():
     """Misuse through the public API that the stand-in must report: a
     buffer freed while a live graph uses it, then that graph launched."""
@@ -118,6 +156,8 @@ def main():
         run_bench(int(sys.argv[2]) if len(sys.argv) > 2 else 10)
     elif what == "model":
         run_model()
+    elif what == "capture":
+        run_capture()
     elif what == "selftest":
         run_selftest()
     else:

@@ -575,6 +575,7 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t stream) {
 
 // ---- report
 int hipstub_violations(void) { return (int)g_violations; }
+int hipstub_recorded(void) { return (int)g_captured; }   // launches recorded into graphs
 void hipstub_report(void) {
     long live_execs = 0, live_dev = 0;
     size_t live_bytes = 0;

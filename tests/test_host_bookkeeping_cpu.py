@@ -14,6 +14,8 @@ Scenarios (tests/hostcheck/drive.py):
   * bench: the call sequence of `bench.py --no-cpu-baseline --no-model`
     (decode set per-call and persistent, per-kernel timing, GEMM tables with
     workspace growth and rotating weight copies) -- must be clean;
+  * capture: the calls that take tokens from the host, made while the caller
+    records a graph -- must be refused with nothing recorded;
   * model: the device-resident forward and batched decode with graph replay
     and re-prefill -- must be clean.
 """
@@ -74,5 +76,11 @@ def test_bench_call_sequence_is_clean(harness):
 
 def test_model_call_sequence_is_clean(harness):
     p = _drive(harness, "model")
+    assert p.returncode == 0, p.stderr[-4000:]
+    assert "0 violations" in p.stderr and "ERROR: AddressSanitizer" not in p.stderr
+
+
+def test_token_calls_are_refused_while_a_graph_is_recorded(harness):
+    p = _drive(harness, "capture")
     assert p.returncode == 0, p.stderr[-4000:]
     assert "0 violations" in p.stderr and "ERROR: AddressSanitizer" not in p.stderr
