@@ -387,6 +387,11 @@ static inline int xl_bk(int p) { return (p == PLAN_X256x256 || p == PLAN_XB256x2
 static inline int pipe_bk(int p) {
     return p == PLAN_P32x64k128s4 || is_pb_plan(p) ? 128 : 64;
 }
+// a plan that reads A as bf16 and takes K (K % 64 == 0); the 32 x 64 ring tiles
+// are not built gated (choose_bf16a_plan)
+static inline bool xb_takes(int p, int K, bool gated) {
+    return is_xb_plan(p) && K % (is_pb_plan(p) ? pipe_bk(p) : 64) == 0 && !(gated && p == PLAN_PB32x64k128);
+}
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -1411,7 +1416,9 @@ static int dispatch_bf16a(int p, float *c, const uint16_t *a, const uint16_t *b,
         case PLAN_XB128x128:    return launch_xl<128, 128, 64, GATED, true>(c, a, b, b2, M, K, N);
         case PLAN_XB256x256s1:  return launch_xl<256, 256, 64, GATED, true, 1>(c, a, b, b2, M, K, N);
         case PLAN_XB64x128:     return launch_xl<64, 128, 64, GATED, true>(c, a, b, b2, M, K, N);
-        case PLAN_PB32x64k128:  return launch_pipe<32, 64, 2, 2, 6, GATED, 128, 2, true>(c, a, b, b2, M, K, N);
+        case PLAN_PB32x64k128:
+            if constexpr (GATED) return QH_EINVAL;
+            else return launch_pipe<32, 64, 2, 2, 6, false, 128, 2, true>(c, a, b, b2, M, K, N);
         case PLAN_PB64x64k128:  return launch_pipe<64, 64, 2, 2, 4, GATED, 128, 2, true>(c, a, b, b2, M, K, N);
         default: return QH_EINVAL;
     }
@@ -1419,6 +1426,9 @@ static int dispatch_bf16a(int p, float *c, const uint16_t *a, const uint16_t *b,
 
 
 // gate|up with bf16 A and bf16 C, on the tiles choose_bf16a_plan picks for it
+static inline bool xbc_takes(int p, int K) {
+    return xb_takes(p, K, true) && p != PLAN_XB256x256k32 && p != PLAN_XB256x256s1;
+}
 static int dispatch_bf16ac(int p, uint16_t *h, const uint16_t *a, const uint16_t *b, const uint16_t *b2, int M, int K,
                            int N) {
     float *c = reinterpret_cast<float *>(h);
@@ -1499,10 +1509,11 @@ static int resolve_plan(Ws &ws, int M, int K, int N, bool gated, bool vec, bool 
     if (!vec && !is_rag_plan(plan)) plan = PLAN_SCALAR64;   // forced plans still need vector-safe inputs
     if (plan == PLAN_GEMV && (M > 4 || (size_t)M * K * 4 > 64 * 1024)) plan = PLAN_T64x64;
     if ((is_pipe_plan(plan) || is_pb_plan(plan)) && (K % pipe_bk(plan)) != 0) plan = PLAN_T64x64;   // whole k stages
-    if (plan == PLAN_X64x64s3 && gated) plan = PLAN_T64x64;   // one B block per wave tile
-    if (is_xl_plan(plan) && ((K % xl_bk(plan)) != 0 ||           // xl copies whole k stages and
-                             (size_t)M * K * 4 >= (1ull << 32) ||   // addresses with 32-bit offsets
-                             (size_t)N * K * 2 >= (1ull << 32)))
+    if ((plan == PLAN_X64x64s3 || plan == PLAN_PB32x64k128) && gated) plan = PLAN_T64x64;   // not built gated
+    if ((is_xl_plan(plan) || is_pb_plan(plan)) &&
+        ((is_xl_plan(plan) && K % xl_bk(plan) != 0) ||              // xl copies whole k stages and
+         (size_t)M * K * 4 >= (1ull << 32) ||                       // addresses with 32-bit offsets
+         (size_t)N * K * 2 >= (1ull << 32)))
         plan = PLAN_T64x64;
     if (is_xb_plan(plan) && !abf_ensure(ws, (size_t)M * K)) {     // no room for the bf16 copy of A
         if (strict) return -QH_ETOOBIG;
@@ -1608,7 +1619,7 @@ static int gemm_bf16a_common(float *c, const uint16_t *a, const uint16_t *b, con
         return QH_EINVAL;
     if ((size_t)M * K * 2 >= (1ull << 32) || (size_t)N * K * 2 >= (1ull << 32)) return QH_ETOOBIG;
     int plan = g_forced_plan;
-    if (!is_xb_plan(plan) || (is_pb_plan(plan) && K % pipe_bk(plan))) plan = choose_bf16a_plan(M, K, N, gated);
+    if (!xb_takes(plan, K, gated)) plan = choose_bf16a_plan(M, K, N, gated);
     g_last_plan = plan;
     return gated ? dispatch_bf16a<true>(plan, c, a, b, b2, M, K, N)
                  : dispatch_bf16a<false>(plan, c, a, b, nullptr, M, K, N);
@@ -1629,7 +1640,7 @@ extern "C" int qh_gemm_gate_up_silu_bf16ac(uint16_t *h, const uint16_t *x, const
     if (!h || !x || !wg || !wu || M <= 0 || N <= 0 || K <= 0 || K % 64 || !aligned16(x) || !aligned16(wg) || !aligned16(wu))
         return QH_EINVAL;
     if ((size_t)M * K * 2 >= (1ull << 32) || (size_t)N * K * 2 >= (1ull << 32)) return QH_ETOOBIG;
-    g_last_plan = choose_bf16a_plan(M, K, N, 1);
+    g_last_plan = xbc_takes(g_forced_plan, K) ? g_forced_plan : choose_bf16a_plan(M, K, N, 1);
     return dispatch_bf16ac(g_last_plan, h, x, wg, wu, M, K, N);
 }
 
@@ -1640,7 +1651,7 @@ extern "C" int qh_gemm_split_bf16a(float *c, const uint16_t *a, const uint16_t *
     *part = nullptr;
     *ks = 0;
     if (!g_inited) return QH_ESTATE;
-    if (M > 0 && N > 0 && K > 0 && c && a && b && K % 128 == 0 && aligned16(a) && aligned16(b) &&
+    if (!g_forced_plan && M > 0 && N > 0 && K > 0 && c && a && b && K % 128 == 0 && aligned16(a) && aligned16(b) &&
         (size_t)N * K * 2 < (1ull << 31)) {
         Ws ws = lib_ws();
         const int s = pipe_slices(M, K, N);

@@ -100,3 +100,38 @@ def test_split(M, K, N, slices):
     else:
         c = cd.download(np.float32, M * N)
     numerics.compare(c, a, b, M, K, N, rows=numerics.pick_rows(M, 40))
+
+
+@pytest.mark.parametrize("plan,K,got", [("xb64x128", 1024, "xb64x128"), ("xb128x128", 192, "xb128x128"),
+                                        ("pb64x64k128", 1024, "pb64x64k128"), ("pb64x64k128", 192, "xb64x128"),
+                                        ("pb32x64k128", 1024, "pb64x64k128"), ("xb256x256s1", 1024, "pb64x64k128"),
+                                        ("narrow", 1024, "pb64x64k128")])
+def test_forced_plans(plan, K, got):
+    """A forced plan reaches the products of the bf16 rows where it is built for
+    them; elsewhere the automatic one runs, and nothing is left split."""
+    L, M, N = runtime.init(), 100, 1024
+    a = rne(oracle.f32_bf16_normal(M * K, 5800 + K, 1.0))
+    b = oracle.bf16_normal(2 * N * K, 5801 + K, 0.02)
+    ad, bd = abi.DeviceBuffer.from_array(a), abi.DeviceBuffer.from_array(b)
+    cd, o = abi.DeviceBuffer(4 * M * N), out16(M * N)
+    part, ks = VP(), ctypes.c_int(-1)
+    abi.gemm_gate_up_silu_bf16a_dev(cd.ptr, ad.ptr, bd.ptr, bd.ptr + 2 * N * K, M, K, N)
+    abi.force_plan(abi.PLANS[plan])
+    try:
+        assert L.qh_gemm_gate_up_silu_bf16ac(VP(o.ptr), VP(ad.ptr), VP(bd.ptr), VP(bd.ptr + 2 * N * K), M, K, N) == 0
+        assert abi.last_plan() == got
+        abi.sync()
+        want = cd.download(np.float32, M * N)
+        bits = o.download(np.uint16, M * N + PAD)
+        h = (bits[:M * N].astype(np.uint32) << 16).view(np.float32)
+        # half a unit of bf16 (2^-8), and fp32 sums of K products in another order
+        assert (np.abs(h - want) <= 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max()).all()
+        assert (bits[M * N:] == 0x7FC1).all()
+        K2 = 2048
+        a2, b2 = (abi.DeviceBuffer.from_array(np.zeros(n, np.uint16)) for n in (M * K2, N * K2))
+        assert L.qh_gemm_split_bf16a(VP(cd.ptr), VP(a2.ptr), VP(b2.ptr), M, K2, N, ctypes.byref(part), ctypes.byref(ks)) == 0
+        assert ks.value == 0
+        abi.sync()
+        assert not cd.download(np.float32, M * N).any()
+    finally:
+        abi.force_plan(0)
