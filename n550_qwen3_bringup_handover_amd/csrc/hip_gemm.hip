@@ -427,11 +427,22 @@ static int choose_bf16a_plan(int M, int K, int N, int gated) {
 // 9.2, 3 x 100 x 100 5.2 -> 4.1).  Not where K makes one stage of edge loads
 // (K < 64), nor aligned with more than one round of 128 x 128 tiles, where the
 // register-staged tiles stay ahead (2000 x 1000 x 3000 30.3 against 36.0 us).
+// The kernel's non-temporal C stores cost most where rows of C share 64-byte
+// pieces (N % 16 != 0), so there, aligned and with few stages, the register-staged
+// tiles stay ahead too: 64 x 64 up to K = 128, or 192 for up to half a round (333 x
+// 96 x 1000 3.8 against 4.1 us, 128 x 184 x 3000 4.8 / 5.0, 2000 x 152 x 300 4.8 / 4.5), and 64 x 128 that make more
+// blocks than one round of 128 x 128, up to a K that grows with their number (1000
+// x 96 x 3000 7.3 / 8.5, 1000 x 456 x 3500 13.1 / 14.7, 1000 x 776 x 3500 18.1 /
+// 17.5).  C stores through the L2 instead made 640 x 904 x 3500 16.8 -> 19.5 us.
 static int choose_rag_plan(int M, int K, int N, int gated, bool vec) {
     if (gated || K < 64 || !rag_fits(M, K, N)) return PLAN_AUTO;
     const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    if (t64 <= 2 * g_cus) return PLAN_R64x64;
-    return (t128 <= g_cus || !vec) ? PLAN_R128x128 : PLAN_AUTO;
+    const long t64x128 = (long)((M + 63) / 64) * ((N + 127) / 128);
+    const bool few = vec && N % 16;
+    if (t64 <= 2 * g_cus) return few && M > 32 && t64x128 < 256 && K <= (t64 <= 128 ? 192 : 128) ? PLAN_AUTO : PLAN_R64x64;
+    if (vec && t128 > g_cus) return PLAN_AUTO;
+    if (few && t128 < 256 && t64x128 >= 256 && K <= 2 * t64x128 - 192) return PLAN_AUTO;
+    return PLAN_R128x128;
 }
 
 static int choose_plan(int M, int K, int N, int gated, bool vec) {

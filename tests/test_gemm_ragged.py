@@ -25,6 +25,12 @@ SHAPES = [(1, 64, 1), (65, 65, 63), (64, 72, 128), (3, 100, 100), (130, 129, 129
     (2000, 1001, 3000, False, "rag128x128"), (16, 63, 128, False, "mfma64x64-scalar"),
     (64, 1001, 512, True, "mfma64x64-scalar"), (64, 40, 512, False, "mfma64x64"),
     (30000, 20001, 64, False, "mfma64x64-scalar"),          # A past 2 GiB
+    # few stages and rows of C that share 64-byte pieces (N % 16 != 0)
+    (333, 72, 1000, False, "mfma64x64"), (333, 184, 1000, False, "mfma64x64"), (333, 200, 1000, False, "rag64x64"),
+    (333, 72, 1008, False, "rag64x64"), (333, 73, 1000, False, "rag64x64"), (700, 120, 1000, False, "mfma64x64"),
+    (700, 136, 1000, False, "rag64x64"), (32, 72, 1000, False, "rag64x64"),
+    (1000, 72, 2040, False, "rag64x64"), (1000, 568, 3000, False, "mfma64x128"), (1000, 584, 3000, False, "rag128x128"),
+    (1000, 72, 3008, False, "rag128x128"), (1000, 73, 3000, False, "rag128x128"), (1000, 72, 4072, False, "rag128x128"),
 ])
 def test_ragged_plan_rule(M, K, N, gated, plan):
     assert abi.plan(M, K, N, gated) == plan
