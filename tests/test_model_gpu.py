@@ -156,7 +156,8 @@ def test_forward_api_steps_like_generate(model):
 
 
 def test_chunked_prefill_matches_two_calls(model):
-    # 130 tokens: generate() prefills in chunks 128 + 2; forward() in 64 + 66
+    # 130 tokens: generate() prefills in one pass; forward() in 64 + 66 (several
+    # passes of generate(): test_prefill_passes_gpu)
     rng = np.random.default_rng(1)
     prompt = rng.integers(0, M.VOCAB, 130).astype(np.int32)
     g = model.generate(prompt, 0)
@@ -165,7 +166,7 @@ def test_chunked_prefill_matches_two_calls(model):
     model.forward(prompt[64:], 64)
     lf = model.logits()
     err = np.abs(lg.astype(np.float64) - lf).max()
-    print(f"chunk split 128+2 vs 64+66: max abs logit diff {err:.3e}", flush=True)
+    print(f"130 in one pass vs 64+66: max abs logit diff {err:.3e}", flush=True)
     assert err <= LOGIT_TOL
     top2 = np.sort(lf)[-2:]
     assert g[0] == int(np.argmax(lf)) or top2[1] - top2[0] < TIE_TOL
@@ -448,16 +449,15 @@ def test_batch_size_limits(model, n_seq):
 
 
 def test_longest_context(blob):
-    """max_seq = 8192, the largest cache (the prefill attention then keeps
-    2 x 8192 scores in 70.7 KB of LDS, past the default 64 KB): an
-    8,180-token prompt prefilled in chunks of 128 and in chunks of 100 gives
-    the same last logits within LOGIT_TOL; 11 decode steps to position 8190
+    """max_seq = 8192, the largest cache: an 8,180-token prompt prefilled in
+    four passes of 2,045 and in chunks of 100 gives the same last logits
+    within LOGIT_TOL; 11 decode steps to position 8190
     follow, and the last step's logits equal a forward of the whole
     sequence."""
     rng = np.random.default_rng(8192)
     prompt = rng.integers(0, M.VOCAB, 8180).astype(np.int32)
     with M.Model(blob, max_seq=8192) as m:
-        toks = m.generate(prompt, 11)                 # prefill in chunks of 128, then 11 steps
+        toks = m.generate(prompt, 11)                 # prefill in four passes, then 11 steps
         l_gen = m.logits()
         assert len(toks) == 12 and np.all((toks >= 0) & (toks < M.VOCAB))
         for p0 in range(0, len(prompt), 100):        # other chunk boundaries
