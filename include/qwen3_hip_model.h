@@ -66,7 +66,11 @@ typedef struct qwen3_hip_model qwen3_hip_model;
 /* Mirrors qwen3_init (SRC/qwen3.c:87-146): parses the blob, uploads every
  * tensor to the device (tile-major matrices are re-laid row-major there) and
  * allocates activations and a KV cache for max_seq positions (0 = 4096;
- * at most 8192).  The blob may be freed after this returns. */
+ * at most 8192).  Device memory: the weights (1.19 GB), 229,376 bytes of KV
+ * cache and 512 of rope tables per position, 53,252 bytes of activations per
+ * token of the longest pass (max_seq tokens, at least 128 and at most 2,048:
+ * 109 MB from there on, whether or not such a prompt comes) and 10 MB of
+ * logits and attention partials.  The blob may be freed after this returns. */
 int qwen3_hip_model_open(qwen3_hip_model **model, const void *blob, size_t size, int max_seq);
 
 void qwen3_hip_model_close(qwen3_hip_model *model);
@@ -76,8 +80,13 @@ int qwen3_hip_model_max_seq(const qwen3_hip_model *model);
 /* Mirrors qwen3_forward_batch (SRC/qwen3.c:455-576): n_token tokens (1 ..
  * 128, the reference's QWEN3_MAX_BATCH) at positions pos0 .. pos0+n_token-1;
  * writes their K/V into the cache and leaves the last token's logits on the
- * device.  Unlike the reference, out-of-range sizes return QWEN3_HIP_EINVAL
- * instead of silently doing nothing. */
+ * device.  One token runs as a decode step, several as a chunk (activations
+ * between the kernels fp32 up to 64 tokens; above, those that a product reads
+ * are stored as the bf16 it would round them to).  Unlike the reference,
+ * out-of-range sizes return QWEN3_HIP_EINVAL instead of silently doing
+ * nothing.  Between qwen3_hip_capture_begin and capture_end this call,
+ * generate and batch_prefill return QWEN3_HIP_ERUNTIME: their tokens come from
+ * the host. */
 int qwen3_hip_model_forward(qwen3_hip_model *model, const int *tokens, int n_token, int pos0);
 
 /* Copy the last logits (vocab floats) to host memory (synchronous). */
@@ -86,8 +95,9 @@ int qwen3_hip_model_logits(qwen3_hip_model *model, float *out);
 /* argmax of the last logits, first index on ties (SRC/ops_scalar.c:57-62). */
 int qwen3_hip_model_argmax(qwen3_hip_model *model, int *token);
 
-/* Greedy generation as SRC/main.c:227-256: prefill of the prompt in chunks
- * of 128, out[0] = argmax of the prefill logits, then n_decode steps, step i
+/* Greedy generation as SRC/main.c:227-256: prefill of the prompt in equal
+ * passes of at most 2,048 tokens (of 128 while a dump callback is set),
+ * out[0] = argmax of the prefill logits, then n_decode steps, step i
  * feeding out[i] at position n_prompt + i and producing out[i + 1].  With
  * stop_at_eos, generation ends after the first EOS (151645 or 151643,
  * SRC/qwen3_config.h:28-30), which is included.  out needs n_decode + 1
@@ -109,7 +119,11 @@ int qwen3_hip_model_set_graph(qwen3_hip_model *model, int on);
  * counterpart in the reference, which has no launches).  On MI355X the
  * persistent launch measured 3% slower (1,720-1,750 against 1,780-1,805
  * tok/s for 128 greedy steps after a 128-token prompt).  Steps whose context
- * exceeds 1,024 positions are per-layer launches in either mode.  Turning it on where
+ * exceeds 1,024 positions are per-layer launches in either mode: their
+ * attention takes twice the position ranges, which the persistent launch does
+ * not, and it measured slower there (702 / 728 / 775 / 991 us a step behind
+ * 1,100 / 1,500 / 2,000 / 3,900 positions against 664 / 667 / 689 / 793).  Turning
+ * it on where
  * the device cannot keep the launch's 256 workgroups resident returns
  * QWEN3_HIP_ENODEV.  qwen3_hip_model_persistent returns the mode. */
 int qwen3_hip_model_set_persistent(qwen3_hip_model *model, int on);
@@ -127,7 +141,11 @@ int qwen3_hip_model_persist_errors(qwen3_hip_model *model, unsigned *flags);
  * "x_after_attn_residual", "post_attn_norm_out", "silu_gate_mul_up",
  * "down_proj_out", "layer_out"; and "logits" (layer -1).  The reference's
  * other names (q/k norm and rope outputs, separate gate/up outputs, the
- * final norm) are fused into kernels here and are not produced.  Each dump
+ * final norm) are fused into kernels here and are not produced.  With a
+ * callback set every forward runs as a chunk with fp32 activations, one token
+ * and more than 64 too: the tensors are those of that path, and the logits
+ * differ from a forward's without a callback by the order of fp32 sums and the
+ * bf16 roundings it flips (1e-2 of logits whose deviation is 0.64).  Each dump
  * synchronises the device; NULL (the default) turns dumping off. */
 typedef void (*qwen3_hip_dump_fn)(void *ctx, int layer, const char *name, const float *data,
                                   size_t n);
@@ -160,8 +178,8 @@ int qwen3_hip_batch_open(qwen3_hip_batch **batch, qwen3_hip_model *model, int n_
 void qwen3_hip_batch_close(qwen3_hip_batch *batch);
 
 /* Prefill sequence seq (0 .. n_seq-1) with n_prompt tokens (1 .. max_ctx-1)
- * at positions 0 .. n_prompt-1, in chunks of 128, replacing whatever the
- * sequence held; its next token is the argmax of the last prompt row's
+ * at positions 0 .. n_prompt-1, in passes as qwen3_hip_model_generate's,
+ * replacing whatever the sequence held; its next token is the argmax of the last prompt row's
  * logits.  Sequences may have prompts of different lengths. */
 int qwen3_hip_batch_prefill(qwen3_hip_batch *batch, int seq, const int *prompt, int n_prompt);
 

@@ -53,7 +53,7 @@ static uint16_t *g_abf = nullptr;
 static size_t g_abf_elems = 0;
 static int g_cus = 256;            // compute units of the device (set at init)
 #define PART_INIT_BYTES ((size_t)32 << 20)
-static float *g_part = nullptr;    // K-slice sums of the skinny, stream and narrow kernels (grown on demand)
+static float *g_part = nullptr;    // K-slice sums of the skinny, stream, narrow and split ring kernels (grown on demand)
 static size_t g_part_bytes = 0;
 // tickets of the narrow kernel's K split, one per 32-column block: zero
 // between calls (each call's last block resets the ones it used)
@@ -339,7 +339,9 @@ static inline int m16_ct(int K, int N) { return K <= 2048 && (N + 15) / 16 > g_c
 // MI355X, graph-replayed over weights that are not in any cache, M = 16: 3072 ->
 // 1024 7.6 -> 6.2 us, 2048 -> 1024 4.7 -> 4.2, 3072 -> 2048 8.0 -> 7.3, 2048 ->
 // 2048 5.8 -> 5.3; at K = 1024 nothing to gain, 3.1 -> 3.1 / 3.2; a second
-// round loses, 2048 -> 2048 on 4 columns 6.8, 3072 -> 3072 on 8 12.3 against 8.6)
+// round loses, 2048 -> 2048 on 4 columns 6.8, 3072 -> 3072 on 8 12.3 against 8.6).
+// Over M = 2 .. 16 and N = 256 .. 2048 0.83 to 0.96 of the time on 16 columns
+// (3072 -> 1024 at M = 2 / 8 5.5 / 5.8 -> 4.9 / 5.1; the least at K = 2048, N = 1536)
 static inline int m16_nq(int K, int N) {
     if (K < 2048) return 1;
     return (N + 3) / 4 <= g_cus ? 4 : (N + 7) / 8 <= g_cus ? 2 : 1;
@@ -395,9 +397,10 @@ static inline bool xb_takes(int p, int K, bool gated) {
 
 static inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-// bf16-A shapes: the smallest tile that makes one round -- a CU takes in its
-// operands at 60 to 70 GB/s whatever the kernel, so what counts is the bytes of
-// a block and that every CU has one.  Measured on MI355X, graph-replayed over
+// bf16-A shapes: the smallest tile that makes one round -- these kernels take
+// in a block's operands at 60 to 70 GB/s a CU (one wait and barrier per stage and
+// few stages; plain loads reach 112 to 142 from the L2s), so what counts is the
+// bytes of a block and that every CU has one.  Measured on MI355X, graph-replayed over
 // weights that are not in any cache, against the 128 x 128 tiles: ring 32 x 64,
 // 128 / 512 x 3072 x 1024 23.8 / 23.6 -> 9.8 / 10.5 us and 128 x 1024 x 4096
 // 11.7 -> 6.4; ring 64 x 64, 256 x 1024 x 4096 13.0 -> 7.7, 1024 x 3072 x 1024
@@ -559,11 +562,11 @@ static int choose_plan(int M, int K, int N, int gated, bool vec) {
         if (!gated && M >= 256 && blocks(64, 128) >= 192 && blocks(64, 128) <= g_cus) return PLAN_X64x128;
         if (!gated && M >= 512 && blocks(128, 128) >= 192 && blocks(128, 128) <= g_cus) return PLAN_X128x128;
         if (!gated && M > 128 && blocks(64, 64) >= 192 && blocks(64, 64) <= g_cus) return PLAN_X64x64s3;
-        // between 512 and 1024 rows the ring tiles below make more than a round,
-        // so the same two tiles with fewer blocks too (weights from HBM, against
-        // the register-staged 64 x 64 tiles: 520 x {1024, 2048, 3072} x 1024
-        // 15.8 / 31.6 / 45.7 -> 8.6 / 17.6 / 23.8 us, 600 x 2048 x 2048 32.2 ->
-        // 20.1 on 64 x 128)
+        // between 512 and 1024 rows, where the ring tiles below end, the same two
+        // tiles with fewer blocks too (weights from HBM, against the
+        // register-staged 64 x 64 tiles: 520 x {1024, 2048, 3072} x 1024
+        // 12.7 / 24.9 / 36.4 -> 7.5 / 13.3 / 17.5 us, 600 x 1024 x 100 12.9 -> 7.3,
+        // 1000 x 64 x 64 3.2 -> 3.2; 600 x 1024 x 2048 11.0 -> 9.6 on 64 x 128)
         if (!gated && M > 512 && M < 1024) {
             if (blocks(64, 64) <= g_cus) return PLAN_X64x64s3;
             if (blocks(64, 128) <= g_cus) return PLAN_X64x128;
@@ -1582,10 +1585,11 @@ static int resolve_plan(Ws &ws, int M, int K, int N, bool gated, bool vec, bool 
 // each, so with few tiles a split shortens the chain; the residual + RMSNorm
 // that follows adds the slices.  Measured on MI355X, graph-replayed, weights
 // from HBM, GEMM and norm against the narrow kernel or one slice of the same
-// tiles: M = 128 o / down 10.6 / 12.3 -> 9.0 / 10.1 us, M = 160 11.7 / 16.0 ->
-// 10.0 / 10.9, M = 256 11.8 / 18.1 -> 10.4 / 13.6, M = 32 down 10.0 -> 8.6.  Up
-// to 64 rows at K = 2048 the narrow kernel stays (7.7 against 8.0 us), up to 16
-// the skinny kernel (16 x 3072 7.1 against 8.2).
+// tiles: M = 128 o / down 10.3 / 11.9 -> 8.8 / 9.4 us, M = 160 11.1 / 13.9 ->
+// 9.6 / 10.0, M = 256 11.5 / 15.2 -> 10.0 / 11.8; down of M = 17 / 24 / 33 / 48 / 64
+// 9.9 / 10.1 / 10.0 / 10.1 / 10.1 -> 8.1 / 8.1 / 8.3 / 8.5 / 8.6.  Up to 64 rows at
+// K = 2048 the narrow kernel stays (7.7 against 8.0 us), up to 16 the skinny
+// kernel (16 x 3072 7.1 against 8.2).
 static int pipe_slices(int M, int K, int N) {
     if (K % 128 || K < 2048 || N > 2048 || M <= 16 || (M <= 64 && K <= 2048)) return 1;
     const long tiles = (long)((M + 31) / 32) * ((N + 63) / 64);

@@ -243,8 +243,8 @@ __global__ __launch_bounds__(NTH) void k_rope_cache(const float *__restrict__ qk
 // wave and tile) and by its chain of dependent loads at short ones.  Measured
 // on MI355X per launch against a VALU kernel with two tokens per block and
 // the scores in LDS: 128 tokens 11.6 -> 8.7 us, the 128-token chunks of an
-// 1,800-token prompt 40.0 -> 17.5 us (+ 4.3 for the merge), one token behind
-// 700 positions 28.2 -> 13.6 (+ 4.0).
+// 1,800-token prompt 40.0 -> 17.5 us (+ 4.3 for the merge); in the one pass such
+// a prompt takes, 167 us.
 #define ATT_LD QM_ATT_PART             // row stride of a partial: 16-byte rows, conflict-free
 #define ATT_KS QM_ATT_KS               // key splits, at most
 
@@ -880,7 +880,8 @@ extern "C" int qm_rows_norm(float *x, const float *r, const uint16_t *emb, const
 // The chunk attention's launch: 16-token blocks (each K and V load feeding two
 // row tiles) of four waves once they fill the CUs, 8-token blocks of eight
 // waves below; the context split over blocks while the grid leaves CUs idle
-// and every wave would walk at least ATT_SPLIT_TILES key tiles.
+// and every wave would walk at least ATT_SPLIT_TILES key tiles.  256: the CUs of
+// the device these lines were measured on.
 #define ATT_SPLIT_TILES 4
 template <bool BF>
 static int attention(const float *qkv, void *out, float *part, float *kc, float *vc, const uint16_t *qn,

@@ -48,7 +48,7 @@ void *qh_stream(void);                                    /* hipStream_t */
  * lda = ldb = K, ldc = N.  A is rounded to bf16 (RNE) on the load path. */
 int qh_gemm(float *c_d, const float *a_d, const uint16_t *b_d,
             int M, int K, int N);
-/* qh_gemm, but when the automatic plan splits K over the skinny kernel's
+/* qh_gemm, but when K is split over the ring tiles' or the skinny kernel's
  * blocks the ks > 1 fp32 slice sums are left in library workspace
  * (*part_d: [ks][M][N]) for the caller to add in slice order instead of a
  * reduction launch; otherwise C is written and *ks = 0.  The partials are

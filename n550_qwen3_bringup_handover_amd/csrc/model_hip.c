@@ -546,7 +546,8 @@ int qwen3_hip_model_forward(qwen3_hip_model *m, const int *tokens, int n_token, 
     if (!rc && n_token == 1 && !m->dump) {
         /* one token is a decode step whose next token the caller picks: five
            launches per layer on the GEMV kernels instead of a chunk's eight
-           (measured on MI355X behind 700 positions: 1,255 -> 655 us a call) */
+           (measured on MI355X behind 700 positions, the copy of the logits
+           included: 1,640 -> 745 to 800 us a call) */
         rc = qh_capturing() ? QWEN3_HIP_ERUNTIME : qm_set_tokens(m->state, tokens, 1, m->state + 1, pos0);
         if (!rc) rc = decode_logits(m, 0, pos0 + 1 > QM_LONG_CTX);
     } else if (!rc) {
@@ -770,7 +771,8 @@ int qwen3_hip_batch_prefill(qwen3_hip_batch *b, int seq, const int *prompt, int 
 }
 
 /* one decode step of every sequence: token tok[s] at position pos[s].  When
- * the o and down projections split K (the skinny kernel at small n), their
+ * the o and down projections split K (the skinny kernel up to 16 sequences,
+ * the ring tiles above 64 and, for down, from 17), their
  * slice sums are added by the residual + RMSNorm kernel that consumes them
  * (the sums a reduction launch would form), one launch fewer each. */
 static int batch_step(qwen3_hip_batch *b) {

@@ -1003,8 +1003,9 @@ __global__ __launch_bounds__(NWV * WAVE) void k_gemm_m16(float *__restrict__ c, 
 // time; a weight load instruction covers COLS rows x 64 NQ contiguous bytes and
 // lands in fragment order, so weights skip LDS.  Bound by the L2s' delivery of
 // A, which every block reads whole: 16 x 3072 fp32 to 256 blocks is 50 MB a
-// launch, about 3 of its 6.2 us (7.6 on 64 blocks of 16 columns, each reading
-// 98 KB of weights too; see m16_nq for the line).
+// launch, 1.4 to 1.8 us at the 112 to 142 GB/s a CU takes in and about 3 of its 6.2
+// us as loaded here (7.6 on 64 blocks of 16 columns, each reading 98 KB of
+// weights too; see m16_nq for the line).
 template <int NWV, int KT, int NQ>
 __global__ __launch_bounds__(NWV * WAVE) void k_gemm_m16q(float *__restrict__ c, const float *__restrict__ a,
                                                           const uint16_t *__restrict__ b, int M, int N) {
